@@ -8,9 +8,9 @@
 //             or four wavefronts: the sweeps of tri_mfma.h.
 //             The 512 rows are what four wavefronts hold beside the factor
 //             tiles in flight (256 registers a lane).  Against the kernel below
-//             at its sizes: potrs 2000 x (149, 16 rhs) 1.13 -> 0.30 ms, getrs
-//             256 x (500, 7 rhs) 1.90 -> 0.25 ms, getrs 8192 x (256, 1 rhs)
-//             1.92 -> 1.28 ms (3.4 TB/s of the factor).
+//             at its sizes: potrs 2000 x (149, 16 rhs) 1.13 -> 0.27 ms, getrs
+//             256 x (500, 7 rhs) 1.90 -> 0.22 ms, getrs 8192 x (256, 1 rhs)
+//             1.92 -> 1.15 ms (3.7 TB/s of the factor).
 //   above     one 256-thread workgroup per matrix, up to 8 right-hand sides in
 //             LDS, one barrier per column.
 //

@@ -8,9 +8,10 @@
 // block feeds the updates of the blocks below it as it is.  W wavefronts hold
 // the blocks cyclically (block t in wavefront t % W); a solved block reaches
 // the other wavefronts through X, the vectors' LDS array, with one barrier per
-// 16 columns.  The 16 x 16 diagonal blocks are solved on the vector unit: the
-// value of a row reaches the four row groups by permlane swaps, a column of
-// the block by DPP row_newbcast from registers.
+// 16 columns.  A 16 x 16 diagonal block is solved four rows at a time: permlane
+// swaps give every lane its vector's four rows, each lane solves the 4 x 4
+// triangle with the factor's entries as scalars, and one MFMA takes the four
+// rows out of the rest of the block.
 //
 // Why: a sweep with one barrier per column (one row per thread, X in LDS)
 // costs a barrier and an LDS round trip per column and right-hand-side pass,
@@ -53,21 +54,24 @@ __device__ __forceinline__ bool tri_fits(long lda, int n) { return lda * n < (1l
 
 namespace tri_detail {
 
-// x of row group G (lanes 16 G .. 16 G + 15) in all four groups
-template <int G>
-__device__ __forceinline__ double group_bcast(double x)
+// the values of x in the four row groups (lanes 16 g .. 16 g + 15), each in all lanes
+__device__ __forceinline__ void group_values(double x, double (&y)[4])
 {
     const long long b = __double_as_longlong(x);
-    unsigned r[2] = {(unsigned)b, (unsigned)(b >> 32)};
+    unsigned r[2] = {(unsigned)b, (unsigned)(b >> 32)}, z[4][2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-        // [x0 x0 x2 x2] and [x1 x1 x3 x3], then one half twice
+        // [x0 x0 x2 x2] and [x1 x1 x3 x3], then each half twice
         const auto p = __builtin_amdgcn_permlane16_swap(r[h], r[h], false, false);
-        const unsigned y = (G & 1) ? p[1] : p[0];
-        const auto q = __builtin_amdgcn_permlane32_swap(y, y, false, false);
-        r[h] = (G & 2) ? q[1] : q[0];
+        const auto e = __builtin_amdgcn_permlane32_swap(p[0], p[0], false, false);
+        const auto o = __builtin_amdgcn_permlane32_swap(p[1], p[1], false, false);
+        z[0][h] = e[0];
+        z[1][h] = o[0];
+        z[2][h] = e[1];
+        z[3][h] = o[1];
     }
-    return __longlong_as_double(((long long)r[1] << 32) | r[0]);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) y[g] = __longlong_as_double(((long long)z[g][1] << 32) | z[g][0]);
 }
 
 __device__ __forceinline__ double lane_value(double x, int lane)
@@ -77,51 +81,41 @@ __device__ __forceinline__ double lane_value(double x, int lane)
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
-// lane S of each row of 16 lanes, in all 16
-template <int S>
-__device__ __forceinline__ double row_lane(double x)
-{
-    return __longlong_as_double(
-        __builtin_amdgcn_update_dpp(0LL, __double_as_longlong(x), 0x150 + S, 0xF, 0xF, true));
-}
-
-// t[i] holds entry (4 i + lk, li); r its reciprocals (kTriReciprocal)
+// Rows 4 S .. 4 S + 3 of the 16 x 16 diagonal block whose A-operand tile is t
+// (t[i] holds entry (li, 4 i + lk)): every lane solves the 4 x 4 triangle for
+// its vector, then one MFMA takes the four rows out of the rows below.
 template <int S, TriDiag DIAG>
-__device__ __forceinline__ void diag_step(d4 &x, const d4 &t, const d4 &r, int lk)
+__device__ __forceinline__ void diag_slice(d4 &x, const d4 &t, int li, int lk)
 {
-    constexpr int IS = S >> 2, G = S & 3;
-    double xs = group_bcast<G>(x[IS]);
-    if constexpr (DIAG == kTriDivide) xs = xs / lane_value(t[IS], 16 * G + S);
-    if constexpr (DIAG == kTriReciprocal) xs = lane_value(r[IS], 16 * G + S) * xs;
+    double y[4];
+    group_values(x[S], y);
+    auto entry = [&](int r, int c) { return lane_value(t[S], 16 * c + 4 * S + r); };
 #pragma unroll
-    for (int i = IS; i < 4; ++i) {
-        const double y = fma(-xs, row_lane<S>(t[i]), x[i]);
-        if (i > IS) {
-            x[i] = y;
-        } else {
-            const double z = lk > G ? y : x[i];
-            x[i] = lk == G ? xs : z;
-        }
+    for (int r = 0; r < 4; ++r) {
+#pragma unroll
+        for (int c = 0; c < r; ++c) y[r] = fma(-y[c], entry(r, c), y[r]);
+        if constexpr (DIAG == kTriDivide) y[r] = y[r] / entry(r, r);
+        if constexpr (DIAG == kTriReciprocal) y[r] = (1.0 / entry(r, r)) * y[r];
     }
+    const double lo = (lk & 1) ? y[1] : y[0], hi = (lk & 1) ? y[3] : y[2];
+    const double own = (lk & 2) ? hi : lo;
+    if constexpr (S < 3) {
+        const double a = li > 4 * S + 3 ? t[S] : 0.0;
+        x = __builtin_amdgcn_mfma_f64_16x16x4f64(a, -own, x, 0, 0, 0);
+    }
+    x[S] = own;
 }
 
-template <int S, TriDiag DIAG>
-__device__ __forceinline__ void diag_steps(d4 &x, const d4 &t, const d4 &r, int lk)
-{
-    diag_step<S, DIAG>(x, t, r, lk);
-    __builtin_amdgcn_sched_barrier(0);          // one column's broadcasts at a time in registers
-    if constexpr (S < 15) diag_steps<S + 1, DIAG>(x, t, r, lk);
-}
-
-// The 16 x 16 diagonal block.
 template <TriDiag DIAG>
-__device__ __forceinline__ void diag_solve(d4 &x, const d4 &t, int lk)
+__device__ __forceinline__ void diag_solve(d4 &x, const d4 &t, int li, int lk)
 {
-    d4 r = t;
-    if constexpr (DIAG == kTriReciprocal)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) r[i] = 1.0 / t[i];
-    diag_steps<0, DIAG>(x, t, r, lk);
+    diag_slice<0, DIAG>(x, t, li, lk);
+    __builtin_amdgcn_sched_barrier(0);          // one slice's scalars at a time in registers
+    diag_slice<1, DIAG>(x, t, li, lk);
+    __builtin_amdgcn_sched_barrier(0);
+    diag_slice<2, DIAG>(x, t, li, lk);
+    __builtin_amdgcn_sched_barrier(0);
+    diag_slice<3, DIAG>(x, t, li, lk);
 }
 
 }  // namespace tri_detail
@@ -146,7 +140,6 @@ __device__ __forceinline__ void tri_sweep(TriView v, int n, double *X)
     // byte steps of a logical row and column, forward
     const int ds = 8 * (v.trans ? (int)v.lda : 1), dk = 8 * (v.trans ? 1 : (int)v.lda);
     const int tile = (rev ? 15 - li : li) * ds + (rev ? 3 - lk : lk) * dk;
-    const int diag = (rev ? 3 - lk : lk) * ds + (rev ? 15 - li : li) * dk;
     auto ld = [&](int lane_off, int off) {
         return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, lane_off, off, 0));
     };
@@ -157,12 +150,8 @@ __device__ __forceinline__ void tri_sweep(TriView v, int n, double *X)
 #pragma unroll
         for (int i = 0; i < 4; ++i) a[i] = ld(tile, at(tr) * ds + (at(tc) + 4 * (rev ? 3 - i : i)) * dk);
     };
-    auto load_diag = [&](int t, d4 &a) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) a[i] = ld(diag, (at(t) + 4 * (rev ? 3 - i : i)) * ds + at(t) * dk);
-    };
     d4 x[NB], av[NB], dt;
-    load_diag(min(w, nt - 1), dt);
+    load_tile(min(w, nt - 1), min(w, nt - 1), dt);
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
         const int t = w + W * b;
@@ -182,7 +171,7 @@ __device__ __forceinline__ void tri_sweep(TriView v, int n, double *X)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int s = 4 * i + lk;
-            if (w == 0 && (s < pad || li < pad)) dt[i] = s == li ? 1.0 : 0.0;
+            if (w == 0 && (s < pad || li < pad)) dt[i] = s == li ? 1.0 : 0.0;      // (li, s)
 #pragma unroll
             for (int b = 0; b < NB; ++b)
                 if (s < pad) av[b][i] = 0.0;
@@ -196,13 +185,21 @@ __device__ __forceinline__ void tri_sweep(TriView v, int n, double *X)
             const int t = t0 + ww;
             if (t >= nt) break;
             if (W == 1 || w == ww) {
-                diag_solve<DIAG>(x[0], dt, lk);
+                if (!rev && 16 * t + 16 > n) {
+                    // rows past n come last: the same there
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int k = 4 * i + lk;
+                        if (16 * t + max(k, li) >= n) dt[i] = k == li ? 1.0 : 0.0;
+                    }
+                }
+                diag_solve<DIAG>(x[0], dt, li, lk);
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int s = 16 * t + 4 * i + lk;
                     if (rev ? s >= pad : s < n) X[xrow(s)] = x[0][i];
                 }
-                if (t + W < nt) load_diag(t + W, dt);
+                if (t + W < nt) load_tile(t + W, t + W, dt);
             }
             if (t + 1 >= nt) break;
             d4 xb;
