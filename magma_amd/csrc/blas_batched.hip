@@ -38,10 +38,15 @@
 #include <cstdint>
 
 #include "kernels.h"
+#include "trsm_vector.h"
 
 namespace magma_amd {
 
 magma_int_t zero_info(int *info, int count, hipStream_t st);
+magma_int_t launch_trsm_mfma(bool left, bool lower, bool trans, bool unit, int m, int n, double alpha, double **A,
+                             int lda, double **B, int ldb, int count, hipStream_t st);
+magma_int_t launch_getri_mfma(int n, double **A, int lda, int **ipiv, double **inv, int ldi, int *info, int count,
+                              hipStream_t st);
 magma_int_t launch_geqrf_reg(int m, int n, double **A, int lda, double **tau, int *info, int count, hipStream_t st);
 
 namespace {
@@ -140,9 +145,7 @@ __global__ void __launch_bounds__(64) trsm_kernel(int m, int n, double alpha, do
         if (id >= count || v >= nv) continue;
         const double *a = A_array[id];
         double *b = B_array[id];
-#define AA(i, j) a[(size_t)(i) + (size_t)(j) * lda]
 #define GV(k) (SIDE == 'L' ? b[(size_t)(k) + (size_t)v * ldb] : b[(size_t)v + (size_t)(k) * ldb])
-#define XV(k) (STAGED ? vec[(size_t)(k) * 64 + lane] : GV(k))
         if (alpha == 0.0) {
             for (int k = 0; k < L; ++k) GV(k) = 0.0;
             continue;
@@ -151,101 +154,12 @@ __global__ void __launch_bounds__(64) trsm_kernel(int m, int n, double alpha, do
 #pragma unroll 8
             for (int k = 0; k < L; ++k) vec[(size_t)k * 64 + lane] = GV(k);
         }
-        if (SIDE == 'L') {
-            if (TRANS == 'N') {
-                if (alpha != 1.0)
-                    #pragma unroll 4
-                    for (int i = 0; i < m; ++i) XV(i) = alpha * XV(i);
-                if (UPLO == 'U') {
-                    for (int k = m - 1; k >= 0; --k) {
-                        double bk = XV(k);
-                        if (bk != 0.0) {
-                            if (!unit) bk = bk / AA(k, k);
-                            XV(k) = bk;
-                            #pragma unroll 4
-                            for (int i = 0; i < k; ++i) XV(i) = fma(-bk, AA(i, k), XV(i));
-                        }
-                    }
-                } else {
-                    for (int k = 0; k < m; ++k) {
-                        double bk = XV(k);
-                        if (bk != 0.0) {
-                            if (!unit) bk = bk / AA(k, k);
-                            XV(k) = bk;
-                            #pragma unroll 4
-                            for (int i = k + 1; i < m; ++i) XV(i) = fma(-bk, AA(i, k), XV(i));
-                        }
-                    }
-                }
-            } else if (UPLO == 'U') {
-                for (int i = 0; i < m; ++i) {
-                    double t = alpha * XV(i);
-                    #pragma unroll 4
-                    for (int k = 0; k < i; ++k) t = fma(-AA(k, i), XV(k), t);
-                    if (!unit) t = t / AA(i, i);
-                    XV(i) = t;
-                }
-            } else {
-                for (int i = m - 1; i >= 0; --i) {
-                    double t = alpha * XV(i);
-                    #pragma unroll 4
-                    for (int k = i + 1; k < m; ++k) t = fma(-AA(k, i), XV(k), t);
-                    if (!unit) t = t / AA(i, i);
-                    XV(i) = t;
-                }
-            }
-        } else if (TRANS == 'N') {
-            if (UPLO == 'U') {
-                for (int j = 0; j < n; ++j) {
-                    double t = XV(j);
-                    if (alpha != 1.0) t = alpha * t;
-                    for (int k = 0; k < j; ++k) {
-                        const double akj = AA(k, j);
-                        if (akj != 0.0) t = fma(-akj, XV(k), t);
-                    }
-                    if (!unit) t = (1.0 / AA(j, j)) * t;
-                    XV(j) = t;
-                }
-            } else {
-                for (int j = n - 1; j >= 0; --j) {
-                    double t = XV(j);
-                    if (alpha != 1.0) t = alpha * t;
-                    for (int k = j + 1; k < n; ++k) {
-                        const double akj = AA(k, j);
-                        if (akj != 0.0) t = fma(-akj, XV(k), t);
-                    }
-                    if (!unit) t = (1.0 / AA(j, j)) * t;
-                    XV(j) = t;
-                }
-            }
-        } else if (UPLO == 'U') {
-            for (int k = n - 1; k >= 0; --k) {
-                double bk = XV(k);
-                if (!unit) bk = (1.0 / AA(k, k)) * bk;
-                for (int j = 0; j < k; ++j) {
-                    const double ajk = AA(j, k);
-                    if (ajk != 0.0) XV(j) = fma(-ajk, bk, XV(j));
-                }
-                if (alpha != 1.0) bk = alpha * bk;
-                XV(k) = bk;
-            }
-        } else {
-            for (int k = 0; k < n; ++k) {
-                double bk = XV(k);
-                if (!unit) bk = (1.0 / AA(k, k)) * bk;
-                for (int j = k + 1; j < n; ++j) {
-                    const double ajk = AA(j, k);
-                    if (ajk != 0.0) XV(j) = fma(-ajk, bk, XV(j));
-                }
-                if (alpha != 1.0) bk = alpha * bk;
-                XV(k) = bk;
-            }
-        }
+        trsm_vector<SIDE, UPLO, TRANS>(m, n, alpha, a, lda, unit, [&](int k) -> double & {
+            return STAGED ? vec[(size_t)k * 64 + lane] : GV(k);
+        });
         if (STAGED)
             for (int k = 0; k < L; ++k) GV(k) = vec[(size_t)k * 64 + lane];
-#undef AA
 #undef GV
-#undef XV
     }
 }
 
@@ -621,6 +535,13 @@ __global__ void __launch_bounds__(256) perm_identity_kernel(int n, double **A_ar
 template <bool T, bool U>
 magma_int_t launch_trsv(int n, double **A, int lda, double **x, int incx, bool unit, int count, hipStream_t st)
 {
+    // from order 17 to 512 the register sweeps, where dtrsv's order is dtrsm's:
+    // 20,000 systems of order 64 448 -> 148 us, of order 32 122 -> 85 us; at
+    // order 8 they take 63 us against 40 us here
+    if (n > 16 && incx == 1 && !(T && !U)) {
+        const magma_int_t r = launch_trsm_mfma(true, !U, T, unit, n, 1, 1.0, A, lda, x, n, count, st);
+        if (r != MAGMA_ERR_NOT_SUPPORTED) return r;
+    }
     int pb = (int)(kTrsvLds / (sizeof(double) * (size_t)n)) - 1;
     pb = std::max(1, std::min(32, pb));
     const size_t lds = sizeof(double) * (size_t)n * (pb + 1);
@@ -641,10 +562,17 @@ magma_int_t launch_trsm(int m, int n, double alpha, double **A, int lda, double 
 {
     const int L = S == 'L' ? m : n, nv = S == 'L' ? n : m;
     // one right-hand side, side Left, alpha 1: dtrsm's loops for NoTrans (both
-    // triangles) and for Trans/Upper are dtrsv's, so the workgroup-per-matrix
-    // trsv kernel gives the same bits with the pivots' columns staged in LDS
+    // triangles) and for Trans/Upper are dtrsv's, so the trsv launch gives the
+    // same bits
     if (S == 'L' && n == 1 && alpha == 1.0 && (T == 'N' || U == 'U') && m <= MAGMA_AMD_TRSV_MAX_N)
         return launch_trsv<T == 'T', U == 'U'>(m, A, lda, B, 1, unit, count, st);
+    if constexpr (!(U == 'L' && (S == 'L') == (T == 'T'))) {
+        // the register sweeps (trsm_mfma.hip) up to order 512: 20,000 x (64, 16
+        // vectors) 1583 -> 188 us
+        const magma_int_t r = launch_trsm_mfma(S == 'L', U == 'L', T == 'T', unit, m, n, alpha, A, lda, B, ldb, count,
+                                               st);
+        if (r != MAGMA_ERR_NOT_SUPPORTED) return r;
+    }
     int G = 1;
     while (G < 64 && G < nv) G *= 2;
     const long items = (long)((count + 64 / G - 1) / (64 / G)) * ((nv + G - 1) / G);
@@ -988,6 +916,10 @@ magma_int_t magma_dgetri_outofplace_batched(magma_int_t n, double **dA_array, ma
         return sync_unless_async(queue);
     }
     if (n > 2048) return MAGMA_ERR_NOT_SUPPORTED;
+    if (n <= 512) {
+        magma_int_t r = launch_getri_mfma(n, dA_array, ldda, dipiv_array, dinvA_array, lddia, info_array, batchCount, st);
+        return r == MAGMA_SUCCESS ? sync_unless_async(queue) : r;
+    }
     perm_identity_kernel<<<persistent_grid(batchCount, 4), 256, sizeof(int) * (size_t)n, st>>>(
         n, dA_array, ldda, dipiv_array, dinvA_array, lddia, info_array, batchCount);
     MAGMA_LAUNCH_CHECK();

@@ -107,3 +107,60 @@ def test_nonfinite_factor_falls_back(queue, oracle, n):
     for s in range(4):
         assert same(X[s], oracle.dgetrs(LU[s], ipiv[s], B[s])), s
     assert np.all(np.isfinite(X[1])) and np.all(np.isfinite(X[2][0]))
+
+
+TRSM = [(s, u, t) for s in "LR" for u in "UL" for t in "NT"]
+
+
+@pytest.mark.parametrize("side,uplo,trans", TRSM)
+@pytest.mark.parametrize("order,nv", [(15, 1), (16, 17), (17, 16), (63, 33), (65, 2), (128, 15), (129, 18), (250, 40),
+                                      (257, 16), (512, 3)])
+def test_trsm_tiles(queue, oracle, side, uplo, trans, order, nv):
+    """Bitwise the oracle's dtrsm at the edges of the tiles and of the kernels'
+    order ranges, unit and non-unit, with NaN where A is not read; matrix 2 has
+    an Inf multiplier, taken or skipped as the reference loops do."""
+    import magma_amd as ma
+    L = ma.load()
+    rng = np.random.default_rng(order * 10 + nv)
+    m, n = (order, nv) if side == "L" else (nv, order)
+    for diag, alpha in (("N", 1.0), ("U", -0.5)):
+        F, _ = factor_batch(rng, 3, order)
+        keep = np.tril(np.ones((order, order), bool), 0 if diag == "N" else -1)
+        A = np.where(keep if uplo == "U" else keep.T, F, np.nan)       # storage is transposed
+        B = rng.uniform(-1, 1, (3, n, m))
+        B[1][:, : m // 2] = 0.0
+        B[2][: n // 2 + 1, :] = 0.0
+        if order > 5:
+            A[2][(5, 2) if uplo == "U" else (2, 5)] = np.inf
+        dA, dB = device(A, order + 1), device(B, m + 2)
+        print(f"trsm tiles {side}{uplo}{trans}{diag} order={order} nv={nv}", flush=True)
+        L.magmablas_dtrsm_batched(ma.MagmaLeft if side == "L" else ma.MagmaRight,
+                                  ma.MagmaUpper if uplo == "U" else ma.MagmaLower,
+                                  ma.MagmaNoTrans if trans == "N" else ma.MagmaTrans,
+                                  ma.MagmaNonUnit if diag == "N" else ma.MagmaUnit, m, n, alpha, dA.ptr, dA.ld,
+                                  dB.ptr, dB.ld, 3, queue.handle)
+        X = dB.numpy()
+        assert bool(dB.t[:, :, m:].isnan().all())
+        for s in range(3):
+            want = oracle.dtrsm(side.encode(), uplo.encode(), trans.encode(), diag.encode(), m, n, alpha, A[s], B[s])
+            assert same(X[s], want), (diag, s)
+
+
+@pytest.mark.parametrize("n", [2, 15, 17, 48, 63, 65, 127, 129, 200, 257, 511])
+def test_getri_tiles(queue, oracle, n):
+    """Bitwise the oracle's dgetrs on the identity; matrix 1 is singular."""
+    import magma_amd as ma
+    import torch
+    rng = np.random.default_rng(n)
+    LU, ipiv = factor_batch(rng, 2, n)
+    LU[1][n // 2, n // 2] = 0.0
+    dA, dI = device(LU, n + 1), ma.DeviceBatch(np.full((2, n, n), 7.0), ld=n + 2)
+    ip = ma.IntBatch(2, n)
+    ip.t.copy_(torch.from_numpy(ipiv))
+    info = torch.full((2,), -1, dtype=torch.int32, device="cuda")
+    print(f"getri tiles n={n}", flush=True)
+    assert ma.load().magma_dgetri_outofplace_batched(n, dA.ptr, dA.ld, ip.ptr, dI.ptr, dI.ld, info.data_ptr(), 2,
+                                                     queue.handle) == 0
+    for s in range(2):
+        assert same(dI.numpy()[s], oracle.dgetrs(LU[s], ipiv[s], np.eye(n))), s
+    assert info.cpu().tolist() == [0, n // 2 + 1]
