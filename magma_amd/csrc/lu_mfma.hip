@@ -1,467 +1,538 @@
-// lu_mfma.hip -- blocked right-looking LU with partial pivoting, FP64, one
-// 256-thread workgroup (4 wavefronts) per matrix, for 64 < max(m, n) <= 512.
+// lu_mfma.hip -- LU with partial pivoting, FP64, 64 < max(m, n) <= 512: one
+// workgroup per matrix, one thread per row, left-looking by block columns of
+// 32 columns.
 //
-// Per panel of PW = 32 columns (rows j0..m-1), three phases separated by
-// workgroup barriers:
+// Rows stay where they are for the whole factorization: a pivot is recorded
+// (pos[row], the row's current logical position, and prow[step], the physical
+// row of a step's pivot) and one last pass puts every column into LAPACK's row
+// order.  Block column p (columns 32 p ..):
 //
-//   panel  The panel lives in registers, row pr = tid + 256 i of it in thread
-//          tid.  Per column: local (|a|, position) key, wavefront arg-max by
-//          DPP (quad, half-row and row mirrors) plus a read of the four row
-//          leaders, then each wavefront's winning row is published in an LDS
-//          slot (double-buffered by column parity) and ONE barrier later every
-//          thread picks the winning wavefront's row as the pivot row.  Row
-//          interchanges inside the panel are logical (pos); rows are written
-//          back to their final positions once, at the end of the panel.
-//   rows   The panel's interchanges as a gather of the 32-row block right of
-//          the panel into LDS, 32 lanes per column (coalesced), the old top
-//          rows stored to the rows they move to; then one thread per column
-//          solves U12 = L11^-1 A12 in registers (L11 from LDS) and leaves -U12
-//          in LDS for the update; then U12 is stored back, 32 lanes per
-//          column.  The columns left of the panel (the L part) take all later
-//          interchanges in one pass after the last panel, a column read and
-//          written once, instead of a gather per panel.
-//   update A22 -= L21 U12 in 32x32 tiles, one tile per wavefront at a time, on
-//          v_mfma_f64_16x16x4f64.  The product is formed transposed
-//          (A22^T -= U12^T L21^T) so the C tile and the L21 operand are read
-//          as contiguous 128-byte column segments; -U12^T comes from LDS.
+//   load    C = A(:, block) into registers in the MFMA result layout, wavefront
+//           w the 16-row tiles w, w + W, ... (issued before the panel of the
+//           block column on its left).
+//   update  for each factored chunk q < p: the chunk's pivot rows of C go to
+//           LDS, two wavefronts solve U = L_qq^-1 C for 16 columns each in
+//           registers (tri_mfma.h), then every wavefront takes C -= L_q U on
+//           v_mfma_f64_16x16x4f64 with its tiles of L_q already in flight.
+//           Rows that are pivots by then are updated too and never looked at.
+//   panel   through LDS into one row per thread.  Per column: the arg-max of
+//           the wavefront (DPP on the high words), its row's key in an LDS
+//           slot, a barrier, the workgroup's pivot from the slots (DPP again),
+//           the pivot row and its reciprocal to LDS, a barrier, and the rank-1
+//           update with the pivot row's entries as DPP operands.
+//   store   the block column, finished U rows included, in physical row order.
+//
+// What bounds it: the chain of a panel column (about 1500 cycles, half of them
+// the two LDS round trips) and, with the chip full, the bytes.  Why
+// left-looking with fixed rows: a right-looking form reads and writes the
+// trailing matrix per panel, moves 64 scattered rows of it, and needs passes of
+// its own for the gather, the U solve and the deferred interchanges of L.  The
+// rows that are already pivots cost MFMA work instead (n^3 in place of 2/3
+// n^3), which has the room.  Why a group of 16 panel columns per loop pass: 32
+// columns unrolled are 70 KB of code, more than the instruction cache.  Why two
+// barriers per column: every wavefront's candidate row written before the
+// first one kept the LDS busy for 450 cycles a column.
+// Measured, getrf alone, right-looking form before: 8192 of order 256 12.85 ms
+// -> 8.88 ms, 256 of order 500 7.5 -> 2.03 ms; 4096 of order 96 0.94 ms (a
+// register-resident kernel for n <= 128) -> 0.67 ms.
 //
 // Replaces the reference's launch chain for these sizes (panel + laswp + trsm
 // + gemm, src/zgetrf_batched.cpp:222-351, src/zgetrf_panel_batched.cpp:127-243,
 // magmablas/zgetf2_kernels.cu:353-760) with one persistent launch.
 //
-// Rounding: every entry receives its updates as single fused multiply-adds
-// in increasing k, in the panel (VALU), the solve (VALU) and the update: the
-// FP64 MFMA applies its four k terms of a slice as the sequential fma chain,
-// slices in increasing k.  Multipliers are a * (1/pivot) (division below
-// DBL_MIN), the pivot is the first maximum of |a| with NaN taken only in the
-// first position.  So factors and pivots are the bits of netlib dgetrf with
-// that update order.  When a multiplier of the panel is not finite the
-// update and solve switch to VALU loops that skip zero U entries as the
-// reference BLAS loops do (only then can the skip change a result).
+// Rounding: every entry receives its updates as single fused multiply-adds in
+// increasing k, in the panel (VALU), the solve and the update: the FP64 MFMA
+// applies its four k terms of a slice as the sequential fma chain, slices in
+// increasing k.  Multipliers are a * (1/pivot) (division below DBL_MIN), the
+// pivot is the first maximum of |a| by logical position with NaN taken only in
+// the first position.  So factors and pivots are the bits of netlib dgetrf with
+// that update order (up to the sign of a zero).  A block column that ends with
+// an entry that is not finite, or meets a pivot below DBL_MIN, is done again from
+// memory with the reference loops, and so are the ones after it: only then can
+// their skip of a zero U entry, or the rule for NaN, change a result.
 #include <cfloat>
 #include <climits>
+#include <type_traits>
 
 #include "kernels.h"
+#include "tri_mfma.h"
 #include "tune.h"
 #include "wave_reduce.h"
 
 namespace magma_amd {
 namespace {
 
-constexpr int kThreads = 256;
-constexpr int kWaves = kThreads / 64;
-constexpr int PW = 32;
-
-typedef double d4 __attribute__((ext_vector_type(4)));
+constexpr int PW = 32;              // columns of a block column
+constexpr int GW = 16;              // columns of a panel group
+constexpr int TPW = 4;              // 16-row tiles per wavefront
 
 __device__ __forceinline__ int pick(const int *arr, int fixed, int id) { return arr ? arr[id] : fixed; }
 
-struct alignas(16) PivSlot {
-    unsigned long long key;   // pivot_key of the wavefront's best row
-    int pos;
-    int pad;
-    double row[PW];           // 16-byte aligned: written in pairs
-};
+// The value with nothing known of how it was computed, so that addresses and
+// masks derived from it are formed where they are used: hoisted out of the
+// loops over block columns and chunks they cost a hundred registers.
+__device__ __forceinline__ GDoublePtr opaque(GDoublePtr p)
+{
+    asm volatile("" : "+v"(p));
+    return p;
+}
+__device__ __forceinline__ int opaque(int x)
+{
+    asm volatile("" : "+v"(x));
+    return x;
+}
 
 template <int MT>
 struct LuSmem {
-    PivSlot slot[2][kWaves];
-    double L11[PW][PW + 1];
-    double Us[PW][MT + 1];    // -U12 of the current panel, [k][column - (j0 + jb)]; the odd
-                              // pitch spreads a column's entries over the banks
-    int src_top[PW];          // logical panel row r came from physical panel row src_top[r]
-    int down_dst[PW];         // physical panel row r (< jb) moves to logical row down_dst[r] (>= jb), or -1
-    int swaps[PW];
-    int pst[MT / PW][PW];     // src_top of every panel, for the deferred left-column interchanges
-    int pdd[MT / PW][PW];     // down_dst of every panel
+    double P[PW][MT + 1];     // the block column by physical row; the odd pitch spreads
+                              // the solve's reads of one row over the banks
+    double U[PW][PW + 1];     // -U of the current chunk, [k][column of the block]
+    alignas(16) double row[PW + 2];     // the pivot row of a panel column, then 1 / pivot
+    int4 slot[MT / 64];       // each wavefront's candidate: |v| low, |v| high + 1, logical, physical row
+    int pos[MT];              // logical position of a physical row
+    int prow[MT];             // physical row of step j's pivot
+    int swaps[PW];            // logical positions of the panel's pivots
 };
 
-template <int MT>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(MT <= 256 ? 2 : 1))) getrf_mfma_kernel(MatSet s)
+// The order of the pivot search: |v| (high word + 1, low word), then the
+// smaller logical position; high word 0 marks a row that is no candidate.
+__device__ __forceinline__ bool before(const int4 &a, const int4 &b)
 {
-    constexpr int RPT = MT / kThreads;
+    if (a.y != b.y) return (unsigned)a.y > (unsigned)b.y;
+    if (a.x != b.x) return (unsigned)a.x > (unsigned)b.x;
+    return a.z < b.z;
+}
+
+// The workgroup's pivot from each thread's candidate: logical position p and
+// physical row pr.  The high words decide it but for ties, which take the
+// longer comparison.  Two barriers with the caller's next one: slot is read
+// after the first and written again after the second.
+template <int W>
+__device__ __forceinline__ void select_pivot(int4 *slot, int4 cand, int w, int &p, int &pr)
+{
+    const int lane = threadIdx.x & 63;
+    const unsigned hk = cand.y;
+    const unsigned mh = wave_max_u32(hk);
+    bool win = hk == mh;
+    if (mh == 0) {
+        win = lane == 0;
+    } else if (__builtin_expect(__builtin_popcountll(__builtin_amdgcn_ballot_w64(win)) != 1, 0)) {
+        const unsigned ml = wave_max_u32(win ? cand.x : 0);
+        win &= (unsigned)cand.x == ml;
+        win &= cand.z == wave_min_i32(win ? cand.z : INT_MAX);
+    }
+    if (win) slot[w] = cand;
+    __syncthreads();
+    const int4 h = slot[lane & (W - 1)];
+    unsigned m = h.y;
+    m = max(m, (unsigned)__builtin_amdgcn_update_dpp(0, (int)m, 0xB1, 0xF, 0xF, false));                // xor 1
+    if (W > 2) m = max(m, (unsigned)__builtin_amdgcn_update_dpp(0, (int)m, 0x4E, 0xF, 0xF, false));     // xor 2
+    if (W > 4) m = max(m, (unsigned)__builtin_amdgcn_update_dpp(0, (int)m, 0x141, 0xF, 0xF, false));    // half-row mirror
+    const unsigned tie = (unsigned)__builtin_amdgcn_ballot_w64((unsigned)h.y == m) & ((1u << W) - 1);
+    int src = __builtin_ctz(tie);
+    if (__builtin_expect((tie & (tie - 1)) != 0, 0)) {
+        int4 best = slot[src];
+#pragma unroll 1
+        for (int q = src + 1; q < W; ++q) {
+            const int4 o = slot[q];
+            if (before(o, best)) {
+                best = o;
+                src = q;
+            }
+        }
+        src = __builtin_amdgcn_readfirstlane(src);
+    }
+    p = __builtin_amdgcn_readlane(h.z, src);
+    pr = __builtin_amdgcn_readlane(h.w, src);
+}
+
+// a += x l, x lane K of nu's 16 lanes (v_fmac_f64 takes it by DPP; every lane
+// of the wavefront must be active)
+template <int K>
+__device__ __forceinline__ void fmac_bcast(double &a, double nu, double l)
+{
+    asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(a) : "v"(nu), "v"(l), "n"(K));
+}
+
+template <int K0, int K1>
+__device__ __forceinline__ void fmac_row(double (&a)[PW], double nu0, double nu1, double l)
+{
+    if constexpr (K0 < K1) {
+        fmac_bcast<(K0 & 15)>(a[K0], K0 < 16 ? nu0 : nu1, l);
+        fmac_row<K0 + 1, K1>(a, nu0, nu1, l);
+    }
+}
+
+// The panel with the reference loops, on P (all threads): columns [0, nc), the
+// first jb factored, skipping zero U entries as reference dger does.
+template <int MT>
+__device__ __forceinline__ void reference_panel(LuSmem<MT> &sm, int m, int j0, int jb, int nc, int &pos,
+                                                int &info)
+{
+    constexpr int W = MT / 64;
+    const int tid = threadIdx.x, w = tid >> 6;
+#pragma unroll 1
+    for (int jj = 0; jj < jb; ++jj) {
+        const int j = j0 + jj;
+        const bool cand = tid < m && pos >= j;
+        const double v = cand ? sm.P[jj][tid] : 0.0;
+        // NaN is the largest in the first position and never taken elsewhere (idamax)
+        unsigned long long key = 0;
+        if (cand && (v == v || pos == j)) key = pivot_key(v == v ? fabs(v) : __builtin_huge_val());
+        const bool top = (key >> 32) != 0;
+        int p, pr;
+        select_pivot<W>(sm.slot, int4{top ? (int)key : 0, cand ? (top ? (int)(key >> 32) + 1 : 1) : 0, pos, tid}, w, p, pr);
+        const double piv = sm.P[jj][pr];
+        if (piv == 0.0 && info == 0) info = j + 1;
+        if (tid == 0) sm.swaps[jj] = p;
+        pos = pos == j ? p : (pos == p ? j : pos);
+        if (tid < m && pos > j) {
+            double l = v;
+            if (piv != 0.0) l = fabs(piv) >= DBL_MIN ? (1.0 / piv) * l : l / piv;
+            sm.P[jj][tid] = l;
+#pragma unroll 1
+            for (int c = jj + 1; c < nc; ++c) {
+                const double u = sm.P[c][pr];
+                if (u != 0.0) sm.P[c][tid] = fma(l, -u, sm.P[c][tid]);
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// A block column with the reference loops, from memory to memory (all
+// threads): the columns' updates by every earlier pivot, then the panel.
+template <int MT>
+__device__ __forceinline__ void reference_block(LuSmem<MT> &sm, GDoublePtr A, long lda, int m, int j0, int jb, int nc,
+                                                int kn, int &pos, int &info)
+{
+    const int tid = threadIdx.x;
+    if (tid < m) {
+#pragma unroll 1
+        for (int c = 0; c < nc; ++c) sm.P[c][tid] = A[(j0 + c) * lda + tid];
+    }
+#pragma unroll 1
+    for (int k = 0; k < kn; ++k) {
+        __syncthreads();
+        if (tid < m && pos > k) {
+            const double l = A[k * lda + tid];
+            const int pr = sm.prow[k];
+#pragma unroll 1
+            for (int c = 0; c < nc; ++c) {
+                const double u = sm.P[c][pr];
+                if (u != 0.0) sm.P[c][tid] = fma(l, -u, sm.P[c][tid]);
+            }
+        }
+    }
+    __syncthreads();
+    reference_panel<MT>(sm, m, j0, jb, nc, pos, info);
+    if (tid < m) {
+#pragma unroll 1
+        for (int c = 0; c < nc; ++c) A[(j0 + c) * lda + tid] = sm.P[c][tid];
+    }
+}
+
+template <int K = 0, class F>
+__device__ __forceinline__ void steps(F f)
+{
+    if constexpr (K < GW) {
+        f(std::integral_constant<int, K>{});
+        steps<K + 1>(f);
+    }
+}
+
+template <int MT>
+__global__ void __launch_bounds__(MT) __attribute__((amdgpu_waves_per_eu(2))) getrf_mfma_kernel(MatSet s)
+{
+    constexpr int W = MT / 64;
     __shared__ LuSmem<MT> sm;
 
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int w = tid >> 6;
-    const int li = lane & 15;
-    const int lk = lane >> 4;
+    int tid = threadIdx.x;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int li = tid & 15;
+    int lk = (tid >> 4) & 3;
     const int cnt = item_count(s);
     const int *idx = item_index(s);
     for (int item = blockIdx.x; item < cnt; item += gridDim.x) {
         const int id = idx ? idx[item] : item;
         const int m = pick(s.m_arr, s.m, id);
         const int n = pick(s.n_arr, s.n, id);
-        const int lda = pick(s.lda_arr, s.lda, id);
-        double *A = s.A[id];
+        const long lda = pick(s.lda_arr, s.lda, id);
+        const GDoublePtr A = (GDoublePtr)s.A[id];
         int *ipiv = s.ipiv[id];
         const int mn = min(m, n);
+        const int npan = (mn + PW - 1) / PW;        // factored chunks
+        const int nblk = (n + PW - 1) / PW;
         int info = 0;
+        bool exact = false;                         // a multiplier or U entry was not finite
+        int pos = tid;
+        __syncthreads();
+        sm.pos[tid] = tid;
+        __syncthreads();
 
-        for (int j0 = 0; j0 < mn; j0 += PW) {
-            const int jb = min(PW, mn - j0);
-            const int mp = m - j0;
-            // ------------------------------------------------ panel --------
-            double a[RPT][PW];
-            int pos[RPT];
+        // 32 columns from c0, a row per thread
+        auto store_rows = [&](int c0, const double (&v)[PW]) {
+            GDoublePtr pa = opaque(A + c0 * lda + tid);
+            if (tid < m) {
 #pragma unroll
-            for (int i = 0; i < RPT; ++i) {
-                const int pr = tid + kThreads * i;
-                pos[i] = pr;
-#pragma unroll
-                for (int c = 0; c < PW; ++c)
-                    a[i][c] = (pr < mp && c < jb) ? A[(j0 + pr) + (size_t)(j0 + c) * lda] : 0.0;
-            }
-            bool bad = false;
-#pragma unroll
-            for (int jj = 0; jj < PW; ++jj) {
-                if (jj < jb) {
-                    // ordered integer keys: |a| + 1 ulp of the bit pattern, 0 for
-                    // rows that are not candidates and for NaN past the first
-                    // position (idamax never takes those)
-                    unsigned long long key = 0;
-                    int kp = INT_MAX;
-                    int own = 0;
-#pragma unroll
-                    for (int i = 0; i < RPT; ++i) {
-                        const int pr = tid + kThreads * i;
-                        const bool cand = pr < mp && pos[i] >= jj;
-                        const double v = a[i][jj];
-                        unsigned long long k2 = 0;
-                        if (cand && (v == v || pos[i] == jj)) k2 = pivot_key(v == v ? fabs(v) : __builtin_huge_val());
-                        const int p2 = cand ? pos[i] : INT_MAX;
-                        if ((k2 > key) || (k2 == key && p2 < kp)) {
-                            key = k2;
-                            kp = p2;
-                            own = i;
-                        }
-                    }
-                    unsigned long long wk = key;
-                    int wp = kp;
-                    wave_argmax_key(wk, wp);
-                    PivSlot &sl = sm.slot[jj & 1][w];
-                    if (wp != INT_MAX && kp == wp) {
-                        // 16-byte stores from the pair holding column jj on
-                        // (the entries left of jj are written too, and unread)
-                        double2 *dst = reinterpret_cast<double2 *>(sl.row);
-#pragma unroll
-                        for (int c = jj & ~1; c < PW; c += 2) {
-                            double v0 = a[0][c], v1 = a[0][c + 1];
-#pragma unroll
-                            for (int i = 1; i < RPT; ++i) {
-                                v0 = (own == i) ? a[i][c] : v0;
-                                v1 = (own == i) ? a[i][c + 1] : v1;
-                            }
-                            dst[c / 2] = make_double2(v0, v1);
-                        }
-                    }
-                    if (lane == 0) {
-                        sl.key = wk;
-                        sl.pos = wp;
-                    }
-                    __syncthreads();
-                    // all four candidates, then the winner's row: two LDS
-                    // round trips, each issued as one batch of reads
-                    unsigned long long ck[kWaves];
-                    int cp[kWaves];
-#pragma unroll
-                    for (int q = 0; q < kWaves; ++q) {
-                        ck[q] = sm.slot[jj & 1][q].key;
-                        cp[q] = sm.slot[jj & 1][q].pos;
-                    }
-                    asm volatile("" ::: "memory");
-                    unsigned long long bk = ck[0];
-                    int bp = cp[0];
-                    int bw = 0;
-#pragma unroll
-                    for (int q = 1; q < kWaves; ++q) {
-                        const bool take = (ck[q] > bk) | ((ck[q] == bk) & (cp[q] < bp));
-                        bk = take ? ck[q] : bk;
-                        bp = take ? cp[q] : bp;
-                        bw = take ? q : bw;
-                    }
-                    const double *prow = sm.slot[jj & 1][bw].row;
-                    // one batch of reads into registers when they fit beside
-                    // the panel (one panel row per thread); else read per use
-                    double u[PW];
-#pragma unroll
-                    for (int c = jj & ~1; c < PW; c += 2) {
-                        const double2 t = reinterpret_cast<const double2 *>(prow)[c / 2];
-                        u[c] = t.x;
-                        u[c + 1] = t.y;
-                    }
-                    if (RPT == 1) asm volatile("" ::: "memory");
-                    const int p = bp;
-                    if (tid == 0) sm.swaps[jj] = p;
-                    const double piv = u[jj];
-                    if (piv == 0.0 && info == 0) info = j0 + jj + 1;
-                    const bool use_rcp = fabs(piv) >= DBL_MIN;
-                    const double rc = 1.0 / piv;
-#pragma unroll
-                    for (int i = 0; i < RPT; ++i) {
-                        const int pr = tid + kThreads * i;
-                        pos[i] = (pos[i] == jj) ? p : ((pos[i] == p) ? jj : pos[i]);
-                        const bool below = pr < mp && pos[i] > jj;
-                        if (below) {
-                            double l = a[i][jj];
-                            if (piv != 0.0) l = use_rcp ? rc * l : l / piv;
-                            a[i][jj] = l;
-                            const bool fin = __builtin_isfinite(l);
-                            bad |= !fin;
-                            if (__builtin_amdgcn_ballot_w64(!fin) == 0) {
-                                // finite multipliers: a zero pivot-row entry adds
-                                // a zero, so the reference dger's skip of it
-                                // changes nothing (up to the sign of a zero)
-#pragma unroll
-                                for (int c = jj + 1; c < PW; ++c) a[i][c] = fma(l, -u[c], a[i][c]);
-                            } else {
-                                // reference dger: a zero pivot-row entry is
-                                // skipped.  fma(0, -0, x) is x exactly, so a zero
-                                // multiplier there leaves the entry as it was.
-                                double ls = l;
-                                asm volatile("" : "+v"(ls));      // keeps the two loops apart
-#pragma unroll
-                                for (int c = jj + 1; c < PW; ++c)
-                                    a[i][c] = fma((u[c] != 0.0) ? ls : 0.0, -u[c], a[i][c]);
-                            }
-                        }
-                    }
+                for (int k = 0; k < PW; ++k) {
+                    if (c0 + k < n) *pa = v[k];
+                    pa += lda;
                 }
             }
-            // panel rows to their final positions; L11, the interchange maps
+        };
+        // this lane's row of tile b, kept inside the matrix for loads
+        int rowc[TPW];
 #pragma unroll
-            for (int i = 0; i < RPT; ++i) {
-                const int pr = tid + kThreads * i;
-                if (pr < mp) {
+        for (int b = 0; b < TPW; ++b) rowc[b] = min(16 * (w + W * b) + li, m - 1);
+        auto live = [&](int b) { return 16 * (w + W * b) < m; };
+        // C: entry (row, column 16 t + lk + 4 i of the block) in c[b][t][i]
+        d4 c[TPW][2];
+        auto load_c = [&](int c0) {
+            GDoublePtr pc = opaque(A + min(c0 + lk, n - 1) * lda);
 #pragma unroll
-                    for (int c = 0; c < PW; ++c)
-                        if (c < jb) A[(j0 + pos[i]) + (size_t)(j0 + c) * lda] = a[i][c];
-                    if (pos[i] < jb) {
+            for (int t = 0; t < 2; ++t)
 #pragma unroll
-                        for (int c = 0; c < PW; ++c) sm.L11[pos[i]][c] = a[i][c];
-                        sm.src_top[pos[i]] = pr;
-                    }
-                    if (pr < jb) sm.down_dst[pr] = (pos[i] >= jb) ? pos[i] : -1;
+                for (int i = 0; i < 4; ++i) {
+#pragma unroll
+                    for (int b = 0; b < TPW; ++b) c[b][t][i] = pc[rowc[b]];
+                    pc += c0 + 16 * t + lk + 4 * i + 4 < n ? 4 * lda : 0;
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+        };
+        // the rows of C from logical position `from` on to P
+        auto tiles_to_p = [&](int from) {
+#pragma unroll
+            for (int b = 0; b < TPW; ++b) {
+                const int row = 16 * (w + W * b) + li;
+                if (row < m && sm.pos[row] >= from) {
+#pragma unroll
+                    for (int t = 0; t < 2; ++t)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) sm.P[16 * t + lk + 4 * i][row] = c[b][t][i];
                 }
             }
-            if (tid < jb) ipiv[j0 + tid] = j0 + sm.swaps[tid] + 1;
-            const bool exact = __syncthreads_or(bad);
-            // src_top entries come from the threads owning the moved rows, in
-            // any wavefront: read them after the barrier
-            if (tid < jb) {
-                sm.pst[j0 / PW][tid] = sm.src_top[tid];
-                sm.pdd[j0 / PW][tid] = sm.down_dst[tid];
-            }
+        };
+        load_c(0);
 
-            // ------------------------------------------------ rows ---------
-            const int cb = j0 + jb;                 // first column right of the panel
-            // Columns right of the panel only: the columns left of it (the L
-            // part) get all later interchanges in one pass after the last
-            // panel.  Three passes over the jb x nright block U12:
-            //   gather  32 consecutive lanes per column (coalesced 256-byte
-            //           reads): logical top row r from panel row src_top[r]
-            //           into Us[r][column], the old top row r to down_dst[r];
-            //           a column's reads all precede its writes (one
-            //           half-wavefront owns it);
-            //   solve   thread per column, U12 = L11^-1 A12 on Us in place
-            //           (stored negated, the update's operand);
-            //   store   32 lanes per column again, U12 back to A.
-            const int nright = n - cb;
-            constexpr int kCPI = kThreads / PW;     // columns per pass of the workgroup
-            constexpr int kBatch = 8;               // passes whose loads are in flight together
-            {
-                const int r = tid & (PW - 1);
-                const int rs = min(r, jb - 1);
-                const int src = sm.src_top[rs];
-                const int dd = (r < jb) ? sm.down_dst[r] : -1;
-#pragma unroll 1
-                for (int cl0 = tid / PW; cl0 < nright; cl0 += kCPI * kBatch) {
-                    double xv[kBatch], wv[kBatch];
-#pragma unroll
-                    for (int u = 0; u < kBatch; ++u) {
-                        const double *col = A + (size_t)(cb + min(cl0 + kCPI * u, nright - 1)) * lda + j0;
-                        xv[u] = col[src];
-                        wv[u] = col[rs];
-                    }
-#pragma unroll
-                    for (int u = 0; u < kBatch; ++u) {
-                        const int cl = cl0 + kCPI * u;
-                        if (cl < nright) {
-                            if (dd >= 0) A[(j0 + dd) + (size_t)(cb + cl) * lda] = wv[u];
-                            sm.Us[r][cl] = (r < jb) ? xv[u] : 0.0;
-                        }
-                    }
-                }
-            }
-            __syncthreads();
-#pragma unroll 1
-            for (int cl = tid; cl < nright; cl += kThreads) {
-                double x[PW];
-#pragma unroll
-                for (int k = 0; k < PW; ++k) x[k] = sm.Us[k][cl];
-                // rows of L11 at and beyond jb are never read for k < jb
-                // into a stored result: x[k] = 0 there
-                if (!exact) {
-#pragma unroll
-                    for (int k = 0; k < PW; ++k) {
-                        const double u = -x[k];
-#pragma unroll
-                        for (int i = k + 1; i < PW; ++i) x[i] = fma(sm.L11[i][k], u, x[i]);
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
-                } else {
-#pragma unroll
-                    for (int k = 0; k < PW; ++k) {
-                        const double u = x[k];
-#pragma unroll
-                        for (int i = k + 1; i < PW; ++i)
-                            if (u != 0.0) x[i] = fma(sm.L11[i][k], -u, x[i]);
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
-                }
-#pragma unroll
-                for (int k = 0; k < PW; ++k) sm.Us[k][cl] = (k < jb) ? -x[k] : -0.0;
-            }
-            __syncthreads();
-            {
-                const int r = tid & (PW - 1);
-                if (r < jb) {
-#pragma unroll 1
-                    for (int cl0 = tid / PW; cl0 < nright; cl0 += kCPI * kBatch) {
-                        double v[kBatch];
-#pragma unroll
-                        for (int u = 0; u < kBatch; ++u) v[u] = sm.Us[r][min(cl0 + kCPI * u, nright - 1)];
-#pragma unroll
-                        for (int u = 0; u < kBatch; ++u)
-                            if (cl0 + kCPI * u < nright) A[(j0 + r) + (size_t)(cb + cl0 + kCPI * u) * lda] = -v[u];
-                    }
-                }
-            }
-            // no barrier: the update reads Us and rows >= cb only
+        for (int p = 0; p < nblk; ++p) {
+            tid = opaque(tid);
+            const int j0 = PW * p;
+            const int jb = min(PW, max(0, mn - j0));
+            const int nc = min(PW, n - j0);
+            const int qn = min(p, npan);
+            bool bad = exact;
 
             // ------------------------------------------------ update -------
-            const int nrt = (m - cb + 31) / 32;
-            const int nct = (n - cb + 31) / 32;
-            if (m > cb && n > cb) {
+            // L_q: entry (row, k = 4 s + lk) in lb[b][s]; the 16 x 16 tiles of
+            // L_qq in pivot order for the wavefronts that solve
+            double lb[TPW][PW / 4];
+            d4 t00, t10, t11;
+            auto load_l = [&](int q, int b0) {
+                GDoublePtr pl = opaque(A + (PW * q + lk) * lda);
+#pragma unroll
+                for (int k = 0; k < PW / 4; ++k) {
+#pragma unroll
+                    for (int b = b0; b < b0 + 2; ++b) lb[b][k] = pl[rowc[b]];
+                    pl += 4 * lda;
+                }
+            };
+            auto load_t = [&](int q) {
+                const int kb = min(PW, mn - PW * q);
+                const int r0 = sm.prow[PW * q + min(li, kb - 1)], r1 = sm.prow[PW * q + min(16 + li, kb - 1)];
+                const GDoublePtr pt = opaque(A + PW * q * lda);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int k = 4 * i + lk;
+                    const GDoublePtr p0 = pt + min(k, kb - 1) * lda;
+                    const GDoublePtr p1 = pt + min(16 + k, kb - 1) * lda;
+                    const double v0 = p0[r0], v1 = p0[r1], v2 = p1[r1];
+                    t00[i] = max(li, k) < kb ? v0 : 0.0;
+                    t10[i] = max(16 + li, k) < kb ? v1 : 0.0;
+                    t11[i] = 16 + max(li, k) < kb ? v2 : 0.0;
+                }
+            };
+            if (qn > 0) {
+                if (w < 2) load_t(0);
+                load_l(0, 0);
+            }
 #pragma unroll 1
-                for (int t = w; t < nrt * nct; t += kWaves) {
-                    const int r0 = cb + 32 * (t % nrt);
-                    const int c0 = cb + 32 * (t / nrt);
-                    if (!exact) {
-                        // D = C^T: lane (lk, li), register i of block (bi, bj)
-                        // holds C(r0 + 16 bj + li, c0 + 16 bi + lk + 4 i)
-                        d4 acc[2][2];
+            for (int q = 0; q < qn; ++q) {
+                const int kb = min(PW, mn - PW * q);
+                li = opaque(li);
+                lk = opaque(lk);
+                // the chunk's pivot rows to P
 #pragma unroll
-                        for (int bi = 0; bi < 2; ++bi)
+                for (int b = 0; b < TPW; ++b) {
+                    const int row = 16 * (w + W * b) + li;
+                    if (row < m && (sm.pos[row] >> 5) == q) {
 #pragma unroll
-                            for (int bj = 0; bj < 2; ++bj)
+                        for (int t = 0; t < 2; ++t)
 #pragma unroll
-                                for (int i = 0; i < 4; ++i) {
-                                    const int row = r0 + 16 * bj + li;
-                                    const int col = c0 + 16 * bi + lk + 4 * i;
-                                    acc[bi][bj][i] = (row < m && col < n) ? A[row + (size_t)col * lda] : 0.0;
-                                }
-#pragma unroll
-                        for (int k0 = 0; k0 < PW; k0 += 4) {
-                            const int kk = k0 + lk;
-                            double ua[2], lb[2];
-#pragma unroll
-                            for (int bi = 0; bi < 2; ++bi) {
-                                const int col = c0 + 16 * bi + li;
-                                ua[bi] = (col < n) ? sm.Us[kk][col - cb] : -0.0;
-                            }
-#pragma unroll
-                            for (int bj = 0; bj < 2; ++bj) {
-                                const int row = r0 + 16 * bj + li;
-                                lb[bj] = (row < m && kk < jb) ? A[row + (size_t)(j0 + kk) * lda] : 0.0;
-                            }
-#pragma unroll
-                            for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-                                for (int bj = 0; bj < 2; ++bj)
-                                    acc[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(ua[bi], lb[bj], acc[bi][bj], 0, 0, 0);
-                        }
-#pragma unroll
-                        for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-                            for (int bj = 0; bj < 2; ++bj)
-#pragma unroll
-                                for (int i = 0; i < 4; ++i) {
-                                    const int row = r0 + 16 * bj + li;
-                                    const int col = c0 + 16 * bi + lk + 4 * i;
-                                    if (row < m && col < n) A[row + (size_t)col * lda] = acc[bi][bj][i];
-                                }
-                    } else {
-                        // reference BLAS loop semantics: skip a zero U entry
-                        for (int e = lane; e < 32 * 32; e += 64) {
-                            const int row = r0 + (e & 31), col = c0 + (e >> 5);
-                            if (row < m && col < n) {
-                                double v = A[row + (size_t)col * lda];
-                                for (int k = 0; k < jb; ++k) {
-                                    const double u = -sm.Us[k][col - cb];
-                                    if (u != 0.0) v = fma(A[row + (size_t)(j0 + k) * lda], -u, v);
-                                }
-                                A[row + (size_t)col * lda] = v;
-                            }
-                        }
+                            for (int i = 0; i < 4; ++i) sm.P[16 * t + lk + 4 * i][row] = c[b][t][i];
                     }
                 }
+                __syncthreads();
+                if (w < 2) {
+                    // lane (lk, li): rows 4 i + lk (x0) and 16 + 4 i + lk (x1) of column 16 w + li
+                    const double *col = sm.P[16 * w + li];
+                    int r0[4], r1[4];
+                    d4 x0, x1;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        r0[i] = sm.prow[PW * q + min(4 * i + lk, kb - 1)];
+                        r1[i] = sm.prow[PW * q + min(16 + 4 * i + lk, kb - 1)];
+                    }
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        x0[i] = 4 * i + lk < kb ? col[r0[i]] : 0.0;
+                        x1[i] = 16 + 4 * i + lk < kb ? col[r1[i]] : 0.0;
+                    }
+                    tri_detail::diag_solve<kTriUnit>(x0, t00, li, lk);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        x1 = __builtin_amdgcn_mfma_f64_16x16x4f64(t10[i], -x0[i], x1, 0, 0, 0);
+                    tri_detail::diag_solve<kTriUnit>(x1, t11, li, lk);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        bad |= !__builtin_isfinite(x0[i]) || !__builtin_isfinite(x1[i]);
+                        sm.U[4 * i + lk][16 * w + li] = -x0[i];
+                        sm.U[16 + 4 * i + lk][16 * w + li] = -x1[i];
+                        if (4 * i + lk < kb) sm.P[16 * w + li][r0[i]] = x0[i];
+                        if (16 + 4 * i + lk < kb) sm.P[16 * w + li][r1[i]] = x1[i];
+                    }
+                    if (q + 1 < qn) load_t(q + 1);
+                }
+                __syncthreads();
+                // a chunk that ends the rows leaves nothing to update
+                if (PW * q + PW < m) {
+                    load_l(q, 2);
+                    double ua[2][PW / 4];
+#pragma unroll
+                    for (int t = 0; t < 2; ++t)
+#pragma unroll
+                        for (int k = 0; k < PW / 4; ++k) ua[t][k] = sm.U[4 * k + lk][16 * t + li];
+#pragma unroll
+                    for (int b = 0; b < TPW; b += 2) {
+                        if (live(b)) {
+#pragma unroll
+                            for (int k = 0; k < PW / 4; ++k)
+#pragma unroll
+                                for (int d = 0; d < 2; ++d)
+#pragma unroll
+                                    for (int t = 0; t < 2; ++t)
+                                        c[b + d][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ua[t][k], lb[b + d][k],
+                                                                                           c[b + d][t], 0, 0, 0);
+                        }
+                        if (b == 0 && q + 1 < qn) load_l(q + 1, 0);
+                    }
+                }
+            }
+
+            // ------------------------------------------------ panel --------
+            // rows that are no pivots yet to P, then a row per thread
+            li = opaque(li);
+            lk = opaque(lk);
+            tiles_to_p(PW * qn);
+            __syncthreads();
+            double a[PW];
+#pragma unroll
+            for (int k = 0; k < PW; ++k) a[k] = sm.P[k][tid];
+            if (p + 1 < nblk) load_c(j0 + PW);
+            const int pos0 = pos, info0 = info;
+            double z = 0.0;                         // NaN when an entry of this row is not finite
+            // GW columns at a time; the rest of the row then moves down to the
+            // front registers, so that the loop's code stays in the
+            // instruction cache (32 columns unrolled: 40 KB)
+#pragma unroll 1
+            for (int g = 0; g < PW; g += GW) {
+                auto step = [&](auto JJ) {
+                    constexpr int jj = JJ;
+                    if (g + jj >= jb) return;
+                    const int j = j0 + g + jj;
+                    const double v = a[jj];
+                    const bool cand = tid < m && pos >= j;
+                    double rv = 1.0 / v;                // beside the search; the pivot's is used
+                    asm volatile("" : "+v"(rv));
+                    // a NaN ends in the finite test below
+                    const long long av = __double_as_longlong(fabs(v));
+                    int pp, pr;
+                    select_pivot<W>(sm.slot, int4{(int)av, cand ? (int)(av >> 32) + 1 : 0, pos, tid}, w, pp, pr);
+                    if (tid == pr) {
+                        double2 *dst = reinterpret_cast<double2 *>(sm.row);
+#pragma unroll
+                        for (int k = jj & ~1; k < PW; k += 2) dst[k / 2] = make_double2(a[k], a[k + 1]);
+                        sm.row[PW] = rv;
+                        sm.swaps[g + jj] = pp;
+                    }
+                    __syncthreads();
+                    const double piv = sm.row[jj], rc = sm.row[PW];
+                    double nu0 = -sm.row[tid & 15], nu1 = -sm.row[16 + (tid & 15)];
+                    asm volatile("s_nop 1" : "+v"(nu0), "+v"(nu1));     // a DPP operand's wait
+                    if (piv == 0.0 && info == 0) info = j + 1;
+                    bad |= piv != 0.0 && !(fabs(piv) >= DBL_MIN);
+                    pos = (pos == j) ? pp : ((pos == pp) ? j : pos);
+                    const bool below = tid < m && pos > j;
+                    double l = piv != 0.0 ? rc * v : v;
+                    a[jj] = below ? l : v;
+                    l = below ? l : 0.0;                // adds a zero where U is finite
+                    fmac_row<jj + 1, PW - GW>(a, nu0, nu1, l);
+                    if (g < GW) fmac_row<PW - GW, PW>(a, nu0, nu1, l);
+                };
+                steps<0>(step);
+#pragma unroll
+                for (int k = 0; k < GW; ++k) {
+                    z = fma(a[k], 0.0, z);
+                    sm.P[g + k][tid] = a[k];
+                }
+#pragma unroll
+                for (int k = 0; k + GW < PW; ++k) a[k] = a[k + GW];
+            }
+            bad |= tid < m && !(z == 0.0);
+            if (__syncthreads_or(bad)) {
+                // the block column is still in A as it was
+                exact = true;
+                pos = pos0;
+                info = info0;
+                reference_block<MT>(sm, A, lda, m, j0, jb, nc, min(j0, mn), pos, info);
+            } else {
+#pragma unroll
+                for (int k = 0; k < PW; ++k) a[k] = sm.P[k][tid];
+                store_rows(j0, a);
+            }
+            if (jb > 0) {
+                sm.pos[tid] = pos;
+                if (tid < m && pos >= j0 && pos < j0 + jb) sm.prow[pos] = tid;
+                if (tid < jb) ipiv[j0 + tid] = sm.swaps[tid] + 1;
             }
             __syncthreads();
         }
-        // Deferred interchanges of the L part: the columns of panel k get the
-        // interchanges of panels k+1, ... in order (each as the panel applied
-        // it: logical top row r from row st[r], old top row r to dd[r]),
-        // through LDS (the U12 staging buffer), with one read and one write
-        // of each column.
-        {
-            const int npan = (mn + PW - 1) / PW;
-            double *buf = &sm.Us[0][0];
-#pragma unroll 1
-            for (int k = 0; k + 1 < npan; ++k) {
-                const int c0 = PW * k, nc = min(PW, mn - c0);
-                const int r0 = PW * (k + 1), nr = m - r0;
-                __syncthreads();
-                for (int e = tid; e < nc * nr; e += kThreads) {
-                    const int cl = e / nr, r = e % nr;
-                    buf[cl * MT + r] = A[(r0 + r) + (size_t)(c0 + cl) * lda];
-                }
-#pragma unroll 1
-                for (int p = k + 1; p < npan; ++p) {
-                    const int off = PW * p - r0, jbp = min(PW, mn - PW * p);
-                    __syncthreads();
-                    constexpr int TPT = PW * PW / kThreads;
-                    double sv[TPT], tv[TPT];
-                    int base[TPT], rr[TPT], dd[TPT];     // base: column cl's row off
+
+        // LAPACK's row order: every column once through P
+        double a[PW];
+        auto load_rows = [&](int c0) {
+            GDoublePtr pa = opaque(A + c0 * lda + min(tid, m - 1));
 #pragma unroll
-                    for (int u = 0; u < TPT; ++u) {
-                        const int e = tid + kThreads * u;
-                        const int cl = e / PW, r = e % PW;
-                        const bool on = cl < nc && r < jbp;
-                        base[u] = on ? cl * MT + off : -1;
-                        rr[u] = r;
-                        dd[u] = on ? sm.pdd[p][r] : -1;
-                        if (on) {
-                            sv[u] = buf[base[u] + sm.pst[p][r]];
-                            tv[u] = buf[base[u] + r];
-                        }
-                    }
-                    __syncthreads();
-#pragma unroll
-                    for (int u = 0; u < TPT; ++u) {
-                        if (base[u] >= 0) {
-                            buf[base[u] + rr[u]] = sv[u];
-                            if (dd[u] >= 0) buf[base[u] + dd[u]] = tv[u];
-                        }
-                    }
-                }
-                __syncthreads();
-                for (int e = tid; e < nc * nr; e += kThreads) {
-                    const int cl = e / nr, r = e % nr;
-                    A[(r0 + r) + (size_t)(c0 + cl) * lda] = buf[cl * MT + r];
-                }
+            for (int k = 0; k < PW; ++k) {
+                a[k] = *pa;
+                pa += c0 + k + 1 < n ? lda : 0;
             }
+        };
+        load_rows(0);
+#pragma unroll 1
+        for (int p = 0; p < nblk; ++p) {
+            const int c0 = PW * p;
+            if (tid < m) {
+#pragma unroll
+                for (int k = 0; k < PW; ++k) sm.P[k][pos] = a[k];
+            }
+            __syncthreads();
+            if (p + 1 < nblk) load_rows(c0 + PW);
+            double o[PW];
+#pragma unroll
+            for (int k = 0; k < PW; ++k) o[k] = sm.P[k][tid];
+            store_rows(c0, o);
+            __syncthreads();
         }
         if (tid == 0) s.info[id] = info;
     }
@@ -470,38 +541,31 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(M
 }  // namespace
 
 template <class K>
-static int resident_per_cu(K kernel)
+static int resident_per_cu(K kernel, int threads)
 {
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, kThreads, 0) != hipSuccess || nb < 1) nb = 1;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, threads, 0) != hipSuccess || nb < 1) nb = 1;
     return nb;
 }
 
-magma_int_t launch_getrf_blocked(const MatSet &s, int max_m, hipStream_t st);
-magma_int_t launch_getrf_reg128(const MatSet &s, int max_dim, int waves_per_simd, hipStream_t st);
+template <int MT>
+static magma_int_t launch_mt(const MatSet &s, int variant, hipStream_t st)
+{
+    const int grid = persistent_grid(s.count, variant == 1 ? 1 : resident_per_cu(getrf_mfma_kernel<MT>, MT));
+    getrf_mfma_kernel<MT><<<grid, MT, 0, st>>>(s);
+    MAGMA_LAUNCH_CHECK();
+    return MAGMA_SUCCESS;
+}
 
-// 64 < max(m, n) <= 512; returns MAGMA_ERR_NOT_SUPPORTED above.  Variant
-// (tuned per size class): 0 as many workgroups per CU as fit, 1 one workgroup
-// per CU, 2 the VALU blocked kernel, 3 / 4 the register-resident kernel
-// (lu_reg128.hip) at three / two wavefronts per SIMD, for max(m, n) <= 128
-// (variant 0 above).
+// 64 < max(m, n) <= 512; returns MAGMA_ERR_NOT_SUPPORTED above.
 magma_int_t launch_getrf_mfma(const MatSet &s, int max_dim, hipStream_t st)
 {
     if (s.count <= 0) return MAGMA_SUCCESS;
     if (max_dim > 512) return MAGMA_ERR_NOT_SUPPORTED;
-    int v = tuned_variant(kTuneGetrf, size_class_of(max_dim));
-    if (v >= 3 && max_dim <= 128) return launch_getrf_reg128(s, max_dim, v == 3 ? 3 : 2, st);
-    if (v >= 3) v = 0;
-    if (v == 2) return launch_getrf_blocked(s, max_dim, st);
-    if (max_dim <= 256) {
-        const int grid = persistent_grid(s.count, v == 1 ? 1 : resident_per_cu(getrf_mfma_kernel<256>));
-        getrf_mfma_kernel<256><<<grid, kThreads, 0, st>>>(s);
-    } else {
-        const int grid = persistent_grid(s.count, v == 1 ? 1 : resident_per_cu(getrf_mfma_kernel<512>));
-        getrf_mfma_kernel<512><<<grid, kThreads, 0, st>>>(s);
-    }
-    MAGMA_LAUNCH_CHECK();
-    return MAGMA_SUCCESS;
+    const int v = tuned_variant(kTuneGetrf, size_class_of(max_dim));
+    if (max_dim <= 128) return launch_mt<128>(s, v, st);
+    if (max_dim <= 256) return launch_mt<256>(s, v, st);
+    return launch_mt<512>(s, v, st);
 }
 
 }  // namespace magma_amd

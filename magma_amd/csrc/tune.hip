@@ -34,7 +34,7 @@ void init_table()
 
 const int kVariants[kTuneFamilies] = {5, 5, 4};
 
-// variants a size class can use: the register-resident LU (3, 4) only up to order 128
+// variants a size class can use: LU variants 3 and 4 only up to order 128
 int class_variants(int f, int c) { return (f == kTuneGetrf && c > 4) ? 3 : kVariants[f]; }
 
 __global__ void fill_kernel(double *p, size_t count, unsigned seed)
@@ -145,7 +145,7 @@ magma_int_t tune_getrf(hipStream_t st, FILE *log)
     const int classes[] = {4, 5, 6};
     const int dims[] = {96, 192, 384};
     const int counts[] = {4096, 2048, 512};
-    const int nv[] = {5, 3, 3};            // the register-resident variants cover n <= 128 only
+    const int nv[] = {2, 2, 2};            // the variants above 1 are names of variant 0
     for (int t = 0; t < 3; ++t) {
         const int n = dims[t], count = counts[t];
         const size_t elems = (size_t)n * n * count;

@@ -1,0 +1,66 @@
+"""LU for 64 < max(m, n) <= 512: orders and shapes at the edges of the 32-column
+blocks, the 16-row tiles and the three kernels' ranges, and matrices that leave
+the fast path (ties, NaN, infinities, overflow, pivots below DBL_MIN) at
+different depths.  Factors, pivots and info are the oracle's bits: every entry
+gets the same fused multiply-adds in the same order, so the tolerance is zero."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(65, 65, 65), (97, 128, 99), (128, 33, 128), (129, 129, 131), (159, 161, 159), (161, 159, 161),
+          (255, 256, 255), (256, 40, 256), (40, 256, 48), (257, 257, 257), (300, 511, 301), (512, 70, 512),
+          (70, 512, 70), (497, 497, 500), (512, 512, 512)]
+
+
+def same(a, b):
+    return a.shape == b.shape and bool(np.all((a == b) | (np.isnan(a) & np.isnan(b))))
+
+
+@pytest.mark.parametrize("m,n,ld", SHAPES)
+def test_getrf_shapes(queue, oracle, m, n, ld):
+    import magma_amd as ma
+    rng = np.random.default_rng(1000 * m + n)
+    A = rng.uniform(-1, 1, (3, n, m))
+    print(f"getrf m={m} n={n} ld={ld}", flush=True)
+    dA = ma.DeviceBatch(A, ld=ld)
+    ret, ipiv, info = ma.dgetrf_batched(dA, queue, m=m, n=n)
+    assert ret == 0
+    got, ip, inf = dA.numpy(), ipiv.numpy(), info.cpu().numpy()
+    for s in range(3):
+        LUo, ipo, info_o = oracle.dgetrf(A[s], m=m, n=n)
+        assert inf[s] == info_o and np.array_equal(ip[s], ipo) and same(got[s], LUo), s
+
+
+@pytest.mark.parametrize("n", [130, 257])
+def test_getrf_special(queue, oracle, n):
+    import magma_amd as ma
+    rng = np.random.default_rng(n)
+    mats = []
+    for t in range(7):
+        A = rng.integers(-2, 3, size=(n, n)).astype(float)      # ties in the pivot search
+        if t == 1:
+            A[:, n // 2] = 0.0
+        if t == 2:
+            A[n - 3] = A[5]
+        if t == 3:
+            A[n // 3, (2 * n) // 3] = np.nan
+        if t == 4:
+            A[7, n - 30], A[n - 9, 40] = np.inf, -np.inf
+        if t == 5:
+            A *= 1e300                                          # overflows during the updates
+        if t == 6:
+            A[:, 33] *= 1e-310                                  # pivots below DBL_MIN
+            A[:, n - 2] *= 1e-312
+        mats.append(A.T.copy())
+    mats.append(np.zeros((n, n)))
+    mats.append(np.eye(n)[::-1].T.copy())
+    A = np.stack(mats)
+    print(f"getrf special n={n}", flush=True)
+    dA = ma.DeviceBatch(A)
+    ret, ipiv, info = ma.dgetrf_batched(dA, queue)
+    assert ret == 0
+    LUo, ipo, info_o = oracle.batch_dgetrf(A)
+    assert np.array_equal(info.cpu().numpy(), info_o)
+    assert np.array_equal(ipiv.numpy(), ipo)
+    assert same(dA.numpy(), LUo)
