@@ -16,7 +16,12 @@
 // MFMA operand layout (v_mfma_f64_16x16x4f64, wave64): lane l supplies
 // A(l%16, l/16) and B(l/16, l%16) of the 16x4 / 4x16 blocks and receives
 // D(l/16 + 4*i, l%16), i = 0..3, of the 16x16 result (FP64 interleaves the
-// result rows, unlike the FP16/FP32 variants' 4*(l/16) + i).
+// result rows, unlike the FP16/FP32 variants' 4*(l/16) + i).  The product is
+// formed transposed (op(B)' as A, op(A)' as B), so a lane's result row index is
+// C's column and a store covers 16 consecutive rows of four columns: 128-byte
+// pieces instead of 32-byte ones (50,000 matrices of orders 8 to 256: 6.07 ->
+// 5.91 ms; with the wavefront-wide search of the tile list and the 16-blocks
+// past C's edge skipped, 5.68 ms).
 #include <type_traits>
 
 #include "kernels.h"
@@ -44,6 +49,23 @@ __device__ __forceinline__ T *global_ptr(T *const *p, int id)
     return (T *)((G const *)p)[id];
 }
 
+// The largest s in [0, count) with prefix[s] <= t (prefix[0] <= t), t uniform
+// over the wavefront: each round all lanes probe, so 50,000 matrices take three
+// dependent loads where halving takes sixteen (a third of a small tile's time).
+__device__ __forceinline__ int tile_owner(const int *prefix, int count, int t)
+{
+    const int lane = threadIdx.x & 63;
+    int lo = 0, hi = count;
+    while (hi - lo > 1) {
+        const int step = (hi - lo + 63) >> 6;
+        const int at = lo + lane * step;
+        const bool le = at < hi && prefix[min(at, count - 1)] <= t;
+        lo += step * (__builtin_popcountll(__builtin_amdgcn_ballot_w64(le)) - 1);
+        hi = min(hi, lo + step);
+    }
+    return lo;
+}
+
 template <bool TA, bool TB, int BT>
 __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(BT == 1 ? 4 : (BT == 2 ? 3 : 2)))) gemm_mfma_kernel(GemmSet g, const int *prefix, int fixed_tiles)
 {
@@ -58,12 +80,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
     for (int t = blockIdx.x * kWaves + wave; t < total; t += stride) {
         int s, local;
         if (prefix) {
-            int lo = 0, hi = g.count;          // largest s with prefix[s] <= t
-            while (hi - lo > 1) {
-                const int mid = (lo + hi) >> 1;
-                if (prefix[mid] <= t) lo = mid; else hi = mid;
-            }
-            s = lo;
+            s = tile_owner(prefix, g.count, t);
             local = t - prefix[s];
         } else {
             s = t / fixed_tiles;
@@ -124,7 +141,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
                 for (int bi = 0; bi < BT; ++bi)
 #pragma unroll
                     for (int bj = 0; bj < BT; ++bj)
-                        acc[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[0][bi][sl], bv[0][bj][sl], acc[bi][bj], 0, 0, 0);
+                        acc[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[0][bj][sl], av[0][bi][sl], acc[bi][bj], 0, 0, 0);
             if (k0 + 16 >= kmain) break;
             if (k0 + 32 < kmain) load16(k0 + 32, av[0], bv[0]);
 #pragma unroll
@@ -133,7 +150,7 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
                 for (int bi = 0; bi < BT; ++bi)
 #pragma unroll
                     for (int bj = 0; bj < BT; ++bj)
-                        acc[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[1][bi][sl], bv[1][bj][sl], acc[bi][bj], 0, 0, 0);
+                        acc[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[1][bj][sl], av[1][bi][sl], acc[bi][bj], 0, 0, 0);
         }
         // tail, 4 k per step in order
         for (int k0 = kmain; k0 < k; k0 += 4) {
@@ -154,17 +171,17 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
             for (int bi = 0; bi < BT; ++bi)
 #pragma unroll
                 for (int bj = 0; bj < BT; ++bj)
-                    acc[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[bi], b[bj], acc[bi][bj], 0, 0, 0);
+                    acc[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[bj], a[bi], acc[bi][bj], 0, 0, 0);
         }
         const double alpha = g.alpha, beta = g.beta;
 #pragma unroll
         for (int bi = 0; bi < BT; ++bi) {
 #pragma unroll
             for (int bj = 0; bj < BT; ++bj) {
-                const int col = col0 + 16 * bj + li;
+                const int row = row0 + 16 * bi + li;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const int row = row0 + 16 * bi + lk + 4 * i;
+                    const int col = col0 + 16 * bj + lk + 4 * i;
                     if (row < m && col < n) {
                         double *c = C + row + (size_t)col * ldc;
                         // beta == 0: C is not read (BLAS semantics)
@@ -195,7 +212,8 @@ gemm_lds_kernel(GemmSet g, const int *prefix, int fixed_tiles)
     __shared__ double Bs[2][kLK][kLPitch];   // [stage][k][column within the tile]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int li = lane & 15, lk = lane >> 4;
-    const int wr = wave & 1, wc = wave >> 1;  // this wavefront's quadrant
+    const int wv = __builtin_amdgcn_readfirstlane(wave);
+    const int wr = wv & 1, wc = wv >> 1;      // this wavefront's quadrant
     // element of a stage each thread moves: A (row ar + 16 j or + 4 j, k ak),
     // B (k bk, column bc), chosen so the global loads are unit-stride
     const int ar = TA ? tid / kLK : tid % kLT, ak = TA ? tid % kLK : tid / kLT;
@@ -207,12 +225,7 @@ gemm_lds_kernel(GemmSet g, const int *prefix, int fixed_tiles)
     for (int t = blockIdx.x; t < total; t += gridDim.x) {
         int s, local;
         if (prefix) {
-            int lo = 0, hi = g.count;          // largest s with prefix[s] <= t
-            while (hi - lo > 1) {
-                const int mid = (lo + hi) >> 1;
-                if (prefix[mid] <= t) lo = mid; else hi = mid;
-            }
-            s = lo;
+            s = tile_owner(prefix, g.count, t);
             local = t - prefix[s];
         } else {
             s = t / fixed_tiles;
@@ -236,6 +249,8 @@ gemm_lds_kernel(GemmSet g, const int *prefix, int fixed_tiles)
             for (int bj = 0; bj < 2; ++bj) acc[bi][bj] = d4{0.0, 0.0, 0.0, 0.0};
 
         const int kmain = k & ~(kLK - 1);
+        // 16-blocks of this wavefront's quadrant inside C
+        const int nbi = (m - row0 - 32 * wr + 15) >> 4, nbj = (n - col0 - 32 * wc + 15) >> 4;
         double ra[4], rb[4];
         auto gload = [&](int kb) {
 #pragma unroll
@@ -263,20 +278,28 @@ gemm_lds_kernel(GemmSet g, const int *prefix, int fixed_tiles)
         for (int kb = 0; kb < kmain; kb += kLK) {
             const bool more = kb + kLK < kmain;
             if (more) gload(kb + kLK);
+            if (nbi > 0 && nbj > 0) {
+                double a[2][4], b[2][4];
 #pragma unroll
-            for (int sl = 0; sl < 4; ++sl) {
-                const int kk = 4 * lk + sl;
-                double a[2], b[2];
+                for (int sl = 0; sl < 4; ++sl) {
+                    const int kk = 4 * lk + sl;
 #pragma unroll
-                for (int q = 0; q < 2; ++q) {
-                    a[q] = As[st][kk][32 * wr + 16 * q + li];
-                    b[q] = Bs[st][kk][32 * wc + 16 * q + li];
+                    for (int q = 0; q < 2; ++q) {
+                        a[q][sl] = As[st][kk][32 * wr + 16 * q + li];
+                        b[q][sl] = Bs[st][kk][32 * wc + 16 * q + li];
+                    }
                 }
+                // blocks past the edge are skipped: a 64 x 64 tile's padding is
+                // a quarter of the work at orders up to 256
 #pragma unroll
                 for (int bi = 0; bi < 2; ++bi)
 #pragma unroll
                     for (int bj = 0; bj < 2; ++bj)
-                        acc[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[bi], b[bj], acc[bi][bj], 0, 0, 0);
+                        if (bi < nbi && bj < nbj) {
+#pragma unroll
+                            for (int sl = 0; sl < 4; ++sl)
+                                acc[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[bj][sl], a[bi][sl], acc[bi][bj], 0, 0, 0);
+                        }
             }
             if (more) sstore(st ^ 1);
             __syncthreads();
@@ -301,17 +324,17 @@ gemm_lds_kernel(GemmSet g, const int *prefix, int fixed_tiles)
             for (int bi = 0; bi < 2; ++bi)
 #pragma unroll
                 for (int bj = 0; bj < 2; ++bj)
-                    acc[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[bi], b[bj], acc[bi][bj], 0, 0, 0);
+                    acc[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[bj], a[bi], acc[bi][bj], 0, 0, 0);
         }
         const double alpha = g.alpha, beta = g.beta;
 #pragma unroll
         for (int bi = 0; bi < 2; ++bi) {
 #pragma unroll
             for (int bj = 0; bj < 2; ++bj) {
-                const int col = col0 + 32 * wc + 16 * bj + li;
+                const int row = row0 + 32 * wr + 16 * bi + li;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const int row = row0 + 32 * wr + 16 * bi + lk + 4 * i;
+                    const int col = col0 + 32 * wc + 16 * bj + lk + 4 * i;
                     if (row < m && col < n) {
                         double *c = C + row + (size_t)col * ldc;
                         // beta == 0: C is not read (BLAS semantics)
