@@ -1,5 +1,5 @@
 // lu_blocked.hip -- blocked right-looking LU and Cholesky, one 256-thread
-// workgroup per matrix, for sizes above the register-resident kernels.
+// workgroup per matrix, for orders above 512.
 //
 // Per panel of PW columns:
 //   panel    the whole workgroup factors rows j0..m-1 x PW columns held in
@@ -475,13 +475,14 @@ magma_int_t launch_getrf_blocked(const MatSet &s, int max_m, hipStream_t st)
     return MAGMA_SUCCESS;
 }
 
+magma_int_t launch_potrf_mfma(const MatSet &s, int max_n, hipStream_t st);
+
 magma_int_t launch_potrf_blocked(const MatSet &s, int max_n, hipStream_t st)
 {
     if (s.count <= 0) return MAGMA_SUCCESS;
+    if (max_n <= 512) return launch_potrf_mfma(s, max_n, st);
     const int grid = s.dev_count ? persistent_grid(s.count, 4) : s.count;
-    if (max_n <= 256)       potrf_blocked_kernel<1, 16><<<grid, kThreads, 0, st>>>(s);
-    else if (max_n <= 512)  potrf_blocked_kernel<2, 16><<<grid, kThreads, 0, st>>>(s);
-    else if (max_n <= 1024) potrf_blocked_kernel<4, 8><<<grid, kThreads, 0, st>>>(s);
+    if (max_n <= 1024) potrf_blocked_kernel<4, 8><<<grid, kThreads, 0, st>>>(s);
     else if (max_n <= 2048) potrf_blocked_kernel<8, 4><<<grid, kThreads, 0, st>>>(s);
     else if (max_n <= 4096) potrf_blocked_kernel<16, 2><<<grid, kThreads, 0, st>>>(s);
     else if (max_n <= 8192) potrf_blocked_kernel<32, 1><<<grid, kThreads, 0, st>>>(s);

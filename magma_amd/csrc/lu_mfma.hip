@@ -54,6 +54,7 @@
 #include <climits>
 #include <type_traits>
 
+#include "dpp_fma.h"
 #include "kernels.h"
 #include "tri_mfma.h"
 #include "tune.h"
@@ -67,20 +68,6 @@ constexpr int GW = 16;              // columns of a panel group
 constexpr int TPW = 4;              // 16-row tiles per wavefront
 
 __device__ __forceinline__ int pick(const int *arr, int fixed, int id) { return arr ? arr[id] : fixed; }
-
-// The value with nothing known of how it was computed, so that addresses and
-// masks derived from it are formed where they are used: hoisted out of the
-// loops over block columns and chunks they cost a hundred registers.
-__device__ __forceinline__ GDoublePtr opaque(GDoublePtr p)
-{
-    asm volatile("" : "+v"(p));
-    return p;
-}
-__device__ __forceinline__ int opaque(int x)
-{
-    asm volatile("" : "+v"(x));
-    return x;
-}
 
 template <int MT>
 struct LuSmem {
@@ -144,23 +131,6 @@ __device__ __forceinline__ void select_pivot(int4 *slot, int4 cand, int w, int &
     }
     p = __builtin_amdgcn_readlane(h.z, src);
     pr = __builtin_amdgcn_readlane(h.w, src);
-}
-
-// a += x l, x lane K of nu's 16 lanes (v_fmac_f64 takes it by DPP; every lane
-// of the wavefront must be active)
-template <int K>
-__device__ __forceinline__ void fmac_bcast(double &a, double nu, double l)
-{
-    asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(a) : "v"(nu), "v"(l), "n"(K));
-}
-
-template <int K0, int K1>
-__device__ __forceinline__ void fmac_row(double (&a)[PW], double nu0, double nu1, double l)
-{
-    if constexpr (K0 < K1) {
-        fmac_bcast<(K0 & 15)>(a[K0], K0 < 16 ? nu0 : nu1, l);
-        fmac_row<K0 + 1, K1>(a, nu0, nu1, l);
-    }
 }
 
 // The panel with the reference loops, on P (all threads): columns [0, nc), the
@@ -468,7 +438,7 @@ __global__ void __launch_bounds__(MT) __attribute__((amdgpu_waves_per_eu(2))) ge
                     __syncthreads();
                     const double piv = sm.row[jj], rc = sm.row[PW];
                     double nu0 = -sm.row[tid & 15], nu1 = -sm.row[16 + (tid & 15)];
-                    asm volatile("s_nop 1" : "+v"(nu0), "+v"(nu1));     // a DPP operand's wait
+                    dpp_operand(nu0, nu1);
                     if (piv == 0.0 && info == 0) info = j + 1;
                     bad |= piv != 0.0 && !(fabs(piv) >= DBL_MIN);
                     pos = (pos == j) ? pp : ((pos == pp) ? j : pos);
