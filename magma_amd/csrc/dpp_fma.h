@@ -15,9 +15,15 @@ __device__ __forceinline__ void fmac_bcast(double &a, double x, double l)
     asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(a) : "v"(x), "v"(l), "n"(K));
 }
 
+template <int K>
+__device__ __forceinline__ void fmac_bcast(float &a, float x, float l)
+{
+    asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(a) : "v"(x), "v"(l), "n"(K));
+}
+
 // a[K] += x[K] l for K0 <= K < K1, x[K] lane K % 16 of x0 (K < 16) or x1
-template <int K0, int K1, int N>
-__device__ __forceinline__ void fmac_row(double (&a)[N], double x0, double x1, double l)
+template <int K0, int K1, int N, class T>
+__device__ __forceinline__ void fmac_row(T (&a)[N], T x0, T x1, T l)
 {
     if constexpr (K0 < K1) {
         fmac_bcast<(K0 & 15)>(a[K0], K0 < 16 ? x0 : x1, l);
@@ -27,7 +33,8 @@ __device__ __forceinline__ void fmac_row(double (&a)[N], double x0, double x1, d
 
 // A DPP operand needs two wait states after a VALU write; the compiler does not
 // look for it inside the asm above.
-__device__ __forceinline__ void dpp_operand(double &x0, double &x1) { asm volatile("s_nop 1" : "+v"(x0), "+v"(x1)); }
+template <class T>
+__device__ __forceinline__ void dpp_operand(T &x0, T &x1) { asm volatile("s_nop 1" : "+v"(x0), "+v"(x1)); }
 
 // lane K of each row of 16 lanes, in all of them
 template <int K>

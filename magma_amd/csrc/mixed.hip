@@ -21,10 +21,10 @@
 //     v_mfma_f32_16x16x16f16 with both operands split hi + lo in FP16 (three
 //     products, FP32 accumulation), computed transposed so that the rows of
 //     C are the fast MFMA index.  Rows already pivoted get a zero L operand.
-//   * the chunk panel (32 columns, all rows) is factored in registers, one
-//     workgroup barrier per column: wavefront arg-max by DPP, each
-//     wavefront publishes its best row in an LDS slot, and every thread picks
-//     the winning slot after the barrier.
+//   * the chunk panel (32 columns, all rows) is factored in registers: per
+//     column the pivot search of pivot_select.h, the pivot row through LDS, and
+//     the rank-1 update with its entries as DPP operands (two barriers; every
+//     wavefront writing its candidate row before a single one was 1% slower).
 //
 // Refinement (all right-hand sides of a group at once, as dsgesv does):
 //   x = 0, r = b; repeat: d = (LU)^-1 r in FP32 (blocked sweeps over the pivot
@@ -45,9 +45,10 @@
 #include <type_traits>
 
 #include "magma_amd.h"
+#include "dpp_fma.h"
 #include "mixed.h"
+#include "pivot_select.h"
 #include "tune.h"
-#include "wave_reduce.h"
 
 namespace magma_amd {
 
@@ -70,14 +71,6 @@ constexpr int CH = 32;          // chunk width
 constexpr int kUPad = CH + 4;   // staging row (halves): 72-byte stride, conflict-free b64 reads
 
 __device__ __forceinline__ int pick(const int *arr, int fixed, int id) { return arr ? arr[id] : fixed; }
-
-struct alignas(16) FSlot {
-    unsigned key;     // pivot_key of the wavefront's best row
-    int cur;
-    int row;
-    int pad;
-    float val[CH];    // 16-byte aligned: written and read four at a time
-};
 
 template <int NMAX, int NB, int RG>
 struct MxSmem {
@@ -105,7 +98,8 @@ struct MxSmem {
     int pivpos[NMAX];     // original row -> pivot position (INT_MAX while unpivoted)
     int cur[NMAX];        // original row -> current position (LAPACK interchange order)
     int cexp[NMAX];       // scaling exponents
-    FSlot slot[2][kWaves];
+    int4 slot[kWaves];               // LU panel: each wavefront's candidate
+    alignas(16) float row[CH + 4];   // and the pivot row, then 1 / pivot
     float ccol[2][CH];    // Cholesky: the published column of the diagonal block
     double red[kWaves];
     int flag;
@@ -457,108 +451,66 @@ struct Mixed {
 #pragma unroll
             for (int cc = 0; cc < CH; ++cc) a[r][cc] = (cc < kb) ? sm.u.f.blk[s0 + cc][o] : 0.0f;
         }
+        static_for<0, CH>([&](auto jc) {
+            constexpr int jj = decltype(jc)::value;
+            if (jj >= kb) return;
+            const int gpos = c0 + s0 + jj;
+            unsigned key = 0;                    // ordered integer key, 0: no candidate
+            int kc = INT_MAX, own = 0;
+            float vo = a[0][jj];
 #pragma unroll
-        for (int jj = 0; jj < CH; ++jj) {
-            if (jj < kb) {
-                const int gpos = c0 + s0 + jj;
-                unsigned key = 0;                    // ordered integer key, 0: no candidate
-                int kc = INT_MAX, own = -1;
-#pragma unroll
-                for (int r = 0; r < RPT; ++r) {
-                    if (act[r]) {
-                        const float v = a[r][jj];
-                        const unsigned k2 = pivot_key((v != v) ? __builtin_huge_valf() : fabsf(v));
-                        const bool take = (k2 > key) | ((k2 == key) & (cur[r] < kc));
-                        key = take ? k2 : key;
-                        kc = take ? cur[r] : kc;
-                        own = take ? r : own;
-                    }
-                }
-                unsigned wk = key;
-                int wc = kc;
-                wave_argmax_key(wk, wc);
-                FSlot &sl = sm.slot[jj & 1][w];
-                if (own >= 0 && kc == wc) {
-                    // 16-byte stores from the quad holding column jj on (the
-                    // entries left of jj are written too, and unread)
-                    float4 *dst = reinterpret_cast<float4 *>(sl.val);
-#pragma unroll
-                    for (int cc = jj & ~3; cc < CH; cc += 4) {
-                        float v[4];
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            v[e] = a[0][cc + e];
-#pragma unroll
-                            for (int r = 1; r < RPT; ++r) v[e] = (own == r) ? a[r][cc + e] : v[e];
-                        }
-                        dst[cc / 4] = make_float4(v[0], v[1], v[2], v[3]);
-                    }
-                    sl.row = tid + kT * own;
-                }
-                if (lane == 0) {
-                    sl.key = wk;
-                    sl.cur = wc;
-                }
-                __syncthreads();
-                // each slot's pivot value is read with the keys, so the
-                // reciprocal starts while the winner's row is in flight
-                unsigned ck[kWaves];
-                int cc4[kWaves];
-                float cv[kWaves];
-#pragma unroll
-                for (int q = 0; q < kWaves; ++q) {
-                    ck[q] = sm.slot[jj & 1][q].key;
-                    cc4[q] = sm.slot[jj & 1][q].cur;
-                    cv[q] = sm.slot[jj & 1][q].val[jj];
-                }
-                asm volatile("" ::: "memory");
-                unsigned bk = ck[0];
-                int bc = cc4[0], bw = 0;
-                float piv = cv[0];
-#pragma unroll
-                for (int q = 1; q < kWaves; ++q) {
-                    const bool take = (ck[q] > bk) | ((ck[q] == bk) & (cc4[q] < bc));
-                    bk = take ? ck[q] : bk;
-                    bc = take ? cc4[q] : bc;
-                    bw = take ? q : bw;
-                    piv = take ? cv[q] : piv;
-                }
-                const float rc = 1.0f / piv;
-                const FSlot &ps = sm.slot[jj & 1][bw];
-                const int prow = ps.row;
-                float u[CH];
-#pragma unroll
-                for (int cc = jj & ~3; cc < CH; cc += 4) {
-                    const float4 t = reinterpret_cast<const float4 *>(ps.val)[cc / 4];
-                    u[cc] = t.x;
-                    u[cc + 1] = t.y;
-                    u[cc + 2] = t.z;
-                    u[cc + 3] = t.w;
-                }
-                asm volatile("" ::: "memory");
-                if (!(piv != 0.0f) || piv != piv) bad = 1;
-                if (tid == 0) {
-                    sm.p[gpos] = prow;
-                    if (ipiv) ipiv[gpos] = bc + 1;
-                }
-#pragma unroll
-                for (int r = 0; r < RPT; ++r) {
-                    const int o = tid + kT * r;
-                    const bool isp = (o == prow);
-                    if (isp) {
-                        act[r] = false;
-                        sm.pivpos[o] = gpos;
-                    }
-                    cur[r] = isp ? gpos : ((cur[r] == gpos) ? bc : cur[r]);
-                    if (act[r] && !bad) {
-                        const float l = a[r][jj] * rc;
-                        a[r][jj] = l;
-#pragma unroll
-                        for (int cc = jj + 1; cc < CH; ++cc) a[r][cc] = fmaf(l, -u[cc], a[r][cc]);
-                    }
+            for (int r = 0; r < RPT; ++r) {
+                if (act[r]) {
+                    const float v = a[r][jj];
+                    const unsigned k2 = pivot_key((v != v) ? __builtin_huge_valf() : fabsf(v));
+                    const bool take = (k2 > key) | ((k2 == key) & (cur[r] < kc));
+                    key = take ? k2 : key;
+                    kc = take ? cur[r] : kc;
+                    own = take ? r : own;
+                    vo = take ? v : vo;
                 }
             }
-        }
+            float rv = 1.0f / vo;                // beside the search; the pivot's is used
+            asm volatile("" : "+v"(rv));
+            int bc, prow;
+            select_pivot<kWaves>(sm.slot, int4{0, (int)key, kc, tid + kT * own}, w, bc, prow);
+            if (tid == (prow & (kT - 1))) {
+                // 16-byte stores from the quad holding column jj on (the
+                // entries left of jj are written too, and unread)
+                float4 *dst = reinterpret_cast<float4 *>(sm.row);
+#pragma unroll
+                for (int cc = jj & ~3; cc < CH; cc += 4) {
+                    float v[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        v[e] = a[0][cc + e];
+#pragma unroll
+                        for (int r = 1; r < RPT; ++r) v[e] = (own == r) ? a[r][cc + e] : v[e];
+                    }
+                    dst[cc / 4] = make_float4(v[0], v[1], v[2], v[3]);
+                }
+                sm.row[CH] = rv;
+                sm.p[gpos] = prow;
+                sm.pivpos[prow] = gpos;
+                if (ipiv) ipiv[gpos] = bc + 1;
+            }
+            __syncthreads();
+            const float piv = sm.row[jj], rc = sm.row[CH];
+            float nu0 = -sm.row[tid & 15], nu1 = -sm.row[16 + (tid & 15)];
+            dpp_operand(nu0, nu1);
+            if (!(piv != 0.0f) || piv != piv) bad = 1;
+#pragma unroll
+            for (int r = 0; r < RPT; ++r) {
+                const bool isp = (tid + kT * r == prow);
+                act[r] &= !isp;
+                cur[r] = isp ? gpos : ((cur[r] == gpos) ? bc : cur[r]);
+                const bool on = act[r] && !bad;
+                float l = a[r][jj] * rc;
+                a[r][jj] = on ? l : a[r][jj];
+                l = on ? l : 0.0f;               // adds a zero where U is finite
+                fmac_row<jj + 1, CH>(a[r], nu0, nu1, l);
+            }
+        });
 #pragma unroll
         for (int r = 0; r < RPT; ++r) {
             const int o = tid + kT * r;
@@ -739,32 +691,66 @@ struct Mixed {
     }
 
     // ---- correction solve: v (FP32, original-row order) := (LU)^-1 v ---------
-    // forward sweep with L (unit for LU), backward sweep with U (for Cholesky
-    // the transposed factor stored above the diagonal)
-    static __device__ __forceinline__ void sweeps(Smem &sm, const float *F, int n, int nr, bool chol)
+    // One sweep over the 32-column chunks of the factorization: forward with L
+    // (unit for LU), backward with U (for Cholesky the transposed factor stored
+    // above the diagonal).  A step's loads do not depend on its values: the
+    // chunk's columns are in flight while the diagonal block is solved, and the
+    // next diagonal block while the columns are applied.  With each loaded where
+    // it is used a step waited for memory twice: 83 us for both sweeps of a
+    // matrix of order 256 among 768, 52 us this way (8192 systems 11.4 -> 10.4
+    // ms).  Prefetching a chunk's L the same way in apply_chunk spilled at three
+    // workgroups per CU and was slower (11.5 ms).
+    template <bool FWD>
+    static __device__ __forceinline__ void sweep(Smem &sm, const float *F, int n, int nr, bool chol)
     {
         const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-        // forward
-#pragma unroll 1
-        for (int kq = 0; kq < n; kq += CH) {
+        const int nch = (n + CH - 1) / CH;
+        constexpr int TPT = CH * CH / kT;       // diagonal block entries per thread
+        float t[TPT];
+        auto load_diag = [&](int kq) {
             const int kb = min(CH, n - kq);
-            for (int e = tid; e < CH * CH; e += kT) {
+#pragma unroll
+            for (int j = 0; j < TPT; ++j) {
                 // consecutive threads: down a column (Cholesky) / along a block row (LU)
+                const int e = tid + kT * j;
                 const int i = chol ? e % CH : e / CH, k = chol ? e / CH : e % CH;
-                float v = 0.0f;
-                if (i < kb && k < kb && k <= i)
-                    v = chol ? F[(kq + i) + (size_t)(kq + k) * n] : F[mixed_diag_offset(n) + 32 * (size_t)kq + CH * i + k];
-                sm.u.s.T[i][k] = v;
+                t[j] = 0.0f;
+                if (i < kb && k < kb && (FWD ? k <= i : k >= i))
+                    t[j] = chol ? F[(kq + i) + (size_t)(kq + k) * n] : F[mixed_diag_offset(n) + 32 * (size_t)kq + CH * i + k];
+            }
+        };
+        load_diag(FWD ? 0 : (nch - 1) * CH);
+#pragma unroll 1
+        for (int s = 0; s < nch; ++s) {
+            const int kq = CH * (FWD ? s : nch - 1 - s);
+            const int kb = min(CH, n - kq);
+#pragma unroll
+            for (int j = 0; j < TPT; ++j) {
+                const int e = tid + kT * j;
+                sm.u.s.T[chol ? e % CH : e / CH][chol ? e / CH : e % CH] = t[j];
+            }
+            // rows still to update
+            bool on[RPT];
+            float f[RPT][CH];
+#pragma unroll
+            for (int r = 0; r < RPT; ++r) {
+                const int o = tid + kT * r;
+                on[r] = s + 1 < nch && o < n && (FWD ? sm.pivpos[o] >= kq + kb : sm.pivpos[o] < kq);
+                if (on[r]) {
+#pragma unroll
+                    for (int k = 0; k < CH; ++k) f[r][k] = (k < kb) ? F[o + (size_t)(kq + k) * n] : 0.0f;
+                }
             }
             __syncthreads();
+            if (s + 1 < nch) load_diag(FWD ? kq + CH : kq - CH);
             // unit-diagonal form: lane i holds row i of the block divided by its
-            // diagonal (Cholesky; LU's L is unit) with the diagonal itself
-            // zeroed, and v_i divided the same way, so each step is one
-            // broadcast and one fma with no lane conditions.  Rows and
-            // columns past kb are zero in T, and v is zero there.
+            // diagonal (LU's L is unit) with the diagonal itself zeroed, and v_i
+            // divided the same way, so each step is one broadcast and one fma
+            // with no lane conditions.  Rows and columns past kb are zero in T,
+            // and v is zero there.
             const int li = lane & (CH - 1);
             const float tdiag = sm.u.s.T[li][li];
-            const float rd = (chol && lane < kb) ? 1.0f / tdiag : 1.0f;
+            const float rd = ((chol || !FWD) && lane < kb) ? 1.0f / tdiag : 1.0f;
             float trow[CH];
 #pragma unroll
             for (int k = 0; k < CH; ++k) trow[k] = (k == li) ? 0.0f : sm.u.s.T[li][k] * rd;
@@ -773,7 +759,8 @@ struct Mixed {
                 const float v0 = sm.u.s.v[g][sm.p[min(kq + lane, NMAX - 1)]];
                 float vi = (lane < kb) ? v0 * rd : 0.0f;
 #pragma unroll
-                for (int k = 0; k < CH; ++k) {
+                for (int k0 = 0; k0 < CH; ++k0) {
+                    const int k = FWD ? k0 : CH - 1 - k0;
                     const float zk = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(vi), k));
                     vi = fmaf(-trow[k], zk, vi);
                 }
@@ -783,76 +770,26 @@ struct Mixed {
                 }
             }
             __syncthreads();
-            if (kq + kb < n) {
-                for (int o = tid; o < n; o += kT) {
-                    if (sm.pivpos[o] >= kq + kb) {
-                        float f[CH];
 #pragma unroll
-                        for (int k = 0; k < CH; ++k) f[k] = (k < kb) ? F[o + (size_t)(kq + k) * n] : 0.0f;
-                        for (int g = 0; g < nr; ++g) {
-                            float acc = sm.u.s.v[g][o];
+            for (int r = 0; r < RPT; ++r) {
+                const int o = tid + kT * r;
+                if (on[r]) {
+                    for (int g = 0; g < nr; ++g) {
+                        float acc = sm.u.s.v[g][o];
 #pragma unroll
-                            for (int k = 0; k < CH; ++k) acc = fmaf(-f[k], sm.u.s.z[g][k], acc);
-                            sm.u.s.v[g][o] = acc;
-                        }
+                        for (int k = 0; k < CH; ++k) acc = fmaf(-f[r][k], sm.u.s.z[g][k], acc);
+                        sm.u.s.v[g][o] = acc;
                     }
                 }
             }
-            __syncthreads();
+            // no barrier: the next step writes T, which was read before the last one
         }
-        // backward, over the same 32-column chunks as the factorization
-#pragma unroll 1
-        for (int kq = ((n - 1) / CH) * CH; kq >= 0; kq -= CH) {
-            const int kb = min(CH, n - kq);
-            for (int e = tid; e < CH * CH; e += kT) {
-                // consecutive threads: down a column (Cholesky) / along a block row (LU)
-                const int i = chol ? e % CH : e / CH, k = chol ? e / CH : e % CH;
-                float v = 0.0f;
-                if (i < kb && k < kb && k >= i)
-                    v = chol ? F[(kq + i) + (size_t)(kq + k) * n] : F[mixed_diag_offset(n) + 32 * (size_t)kq + CH * i + k];
-                sm.u.s.T[i][k] = v;
-            }
-            __syncthreads();
-            // unit-diagonal form as in the forward sweep (U and L^T have
-            // non-unit diagonals in both kinds)
-            const int li = lane & (CH - 1);
-            const float tdiag = sm.u.s.T[li][li];
-            const float rd = (lane < kb) ? 1.0f / tdiag : 1.0f;
-            float trow[CH];
-#pragma unroll
-            for (int k = 0; k < CH; ++k) trow[k] = (k == li) ? 0.0f : sm.u.s.T[li][k] * rd;
-            asm volatile("" ::: "memory");
-            for (int g = w; g < nr; g += kWaves) {
-                const float v0 = sm.u.s.v[g][sm.p[min(kq + lane, NMAX - 1)]];
-                float vi = (lane < kb) ? v0 * rd : 0.0f;
-#pragma unroll
-                for (int k = CH - 1; k >= 0; --k) {
-                    const float yk = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(vi), k));
-                    vi = fmaf(-trow[k], yk, vi);
-                }
-                if (lane < kb) {
-                    sm.u.s.z[g][lane] = vi;
-                    sm.u.s.v[g][sm.p[kq + lane]] = vi;
-                }
-            }
-            __syncthreads();
-            if (kq > 0) {
-                for (int o = tid; o < n; o += kT) {
-                    if (sm.pivpos[o] < kq) {
-                        float f[CH];
-#pragma unroll
-                        for (int k = 0; k < CH; ++k) f[k] = (k < kb) ? F[o + (size_t)(kq + k) * n] : 0.0f;
-                        for (int g = 0; g < nr; ++g) {
-                            float acc = sm.u.s.v[g][o];
-#pragma unroll
-                            for (int k = 0; k < CH; ++k) acc = fmaf(-f[k], sm.u.s.z[g][k], acc);
-                            sm.u.s.v[g][o] = acc;
-                        }
-                    }
-                }
-            }
-            __syncthreads();
-        }
+        __syncthreads();
+    }
+    static __device__ __forceinline__ void sweeps(Smem &sm, const float *F, int n, int nr, bool chol)
+    {
+        sweep<true>(sm, F, n, nr, chol);
+        sweep<false>(sm, F, n, nr, chol);
     }
 
     // ---- refinement of one group of right-hand sides; returns iters or status --
