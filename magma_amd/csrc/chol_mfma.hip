@@ -16,7 +16,7 @@
 // What bounds it: the panel's chain, about 350 cycles a column (square root,
 // reciprocal, the first update), and below it the bytes.  The form before, a
 // right-looking panel of 16 columns with three barriers per column and the
-// trailing matrix rewritten per panel: 2000 of order 149 0.606 -> 0.437 ms, 4096 of
+// trailing matrix rewritten per panel: 2000 of order 149 0.606 -> 0.383 ms, 4096 of
 // order 128 0.849 -> 0.354 ms, 256 of order 512 3.57 -> 0.95 ms, one of order 256
 // 0.42 -> 0.135 ms.
 //
@@ -41,7 +41,6 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 
 constexpr int PW = 32;              // columns of a block column
 constexpr int TPW = 4;              // 16-row tiles per wavefront
-constexpr int KS = 16;              // columns of L per update step
 
 __device__ __forceinline__ int pick(const int *arr, int fixed, int id) { return arr ? arr[id] : fixed; }
 
@@ -74,10 +73,76 @@ __device__ __forceinline__ void panel_columns(double (&d0)[16], double (&d1)[PW]
     }
 }
 
+// Column K of the left half of the panel: the diagonal block's rows d0 (li) and
+// d1 (16 + li), and this thread's row a.
+template <int K>
+__device__ __forceinline__ void left_columns(double (&d0)[16], double (&d1)[16], double (&a)[16], int row, int nb,
+                                             int &fail)
+{
+    if constexpr (K < 16) {
+        const double dkk = row_bcast<K>(d0[K]);
+        if (K < nb && !(dkk > 0.0)) fail = min(fail, K);
+        const double ljj = sqrt(dkk), rc = 1.0 / ljj;
+        d0[K] = rc * d0[K];
+        d1[K] = rc * d1[K];
+        double x0 = -d0[K], x1 = x0;
+        const double l = rc * a[K];
+        a[K] = row == K ? ljj : l;
+        dpp_operand(x0, x1);
+        fmac_row<K + 1, 16>(d0, x0, x0, d0[K]);
+        fmac_row<K + 1, 16>(d1, x0, x0, d1[K]);
+        fmac_row<K + 1, 16>(a, x0, x0, l);
+        left_columns<K + 1>(d0, d1, a, row, nb, fail);
+    }
+}
+
+// Column K of the left half taken from the right half: e the rows 16 + li, b this
+// thread's row, d1 and a their entries in the left half.
+template <int K>
+__device__ __forceinline__ void apply_columns(double (&e)[16], double (&b)[16], const double (&d1)[16],
+                                              const double (&a)[16])
+{
+    if constexpr (K < 16) {
+        double x = -d1[K], y = x;
+        dpp_operand(x, y);
+        fmac_row<0, 16>(e, x, x, d1[K]);
+        fmac_row<0, 16>(b, x, x, a[K]);
+        apply_columns<K + 1>(e, b, d1, a);
+    }
+}
+
+// Column 16 + K.
+template <int K>
+__device__ __forceinline__ void right_columns(double (&e)[16], double (&b)[16], int row, int nb, int &fail)
+{
+    if constexpr (K < 16) {
+        const double dkk = row_bcast<K>(e[K]);
+        if (16 + K < nb && !(dkk > 0.0)) fail = min(fail, 16 + K);
+        const double ljj = sqrt(dkk), rc = 1.0 / ljj;
+        e[K] = rc * e[K];
+        double x = -e[K], y = x;
+        const double l = rc * b[K];
+        b[K] = row == 16 + K ? ljj : l;
+        dpp_operand(x, y);
+        fmac_row<K + 1, 16>(e, x, x, e[K]);
+        fmac_row<K + 1, 16>(b, x, x, l);
+        right_columns<K + 1>(e, b, row, nb, fail);
+    }
+}
+
+// At 192 rows the LDS leaves room for three workgroups per CU but 206 registers
+// only for two: there the panel goes in two halves of 16 columns and the update
+// in steps of 8, which takes 152 (2000 of order 149 0.437 -> 0.383 ms, of order
+// 192 0.530 -> 0.472 ms).  At 128, 256 and 512 rows the LDS holds no more
+// wavefronts than two per SIMD anyway, and the halves cost 3%.
+template <int MT> constexpr bool three_per_simd() { return MT == 192; }
+
 template <int MT>
-__global__ void __launch_bounds__(MT) __attribute__((amdgpu_waves_per_eu(2))) potrf_mfma_kernel(MatSet s)
+__global__ void __launch_bounds__(MT) __attribute__((amdgpu_waves_per_eu(three_per_simd<MT>() ? 3 : 2))) potrf_mfma_kernel(MatSet s)
 {
     constexpr int W = MT / 64;
+    constexpr bool HALVES = three_per_simd<MT>();
+    constexpr int KS = HALVES ? 8 : 16;         // columns of L per update step
     __shared__ double P[PW][MT + 1];
     __shared__ int failed;
 
@@ -173,24 +238,58 @@ __global__ void __launch_bounds__(MT) __attribute__((amdgpu_waves_per_eu(2))) po
             }
             __syncthreads();
             if (64 * w + 64 > j0 && 64 * w < n) {       // wavefronts with a row of the block column
-                double a[PW], d0[16], d1[PW];
-                const int q0 = min(j0 + li, n - 1), q1 = min(j0 + 16 + li, n - 1);
-#pragma unroll
-                for (int k = 0; k < PW; ++k) {
-                    a[k] = P[k][tid];
-                    d1[k] = P[k][q1];
-                    if (k < 16) d0[k] = P[k][q0];
-                }
                 int fail = PW;
-                panel_columns<0>(d0, d1, a, tid - j0, nb, fail);
-                if (fail < PW) failed = fail;           // the same in every wavefront
-                const int kn = min(nb, fail);
-                GDoublePtr pa = opaque(A + j0 * lda + tid);
+                if constexpr (HALVES) {
+                    double a[16], b[16], d1[16], e[16];
+                    const int q0 = min(j0 + li, n - 1), q1 = min(j0 + 16 + li, n - 1);
+                    {
+                        double d0[16];
 #pragma unroll
-                for (int k = 0; k < PW; ++k) {
-                    if (tid < n && tid >= j0 + k && k < kn) *pa = a[k];
-                    pa += lda;
+                        for (int k = 0; k < 16; ++k) {
+                            a[k] = P[k][tid];
+                            d0[k] = P[k][q0];
+                            d1[k] = P[k][q1];
+                        }
+                        left_columns<0>(d0, d1, a, tid - j0, nb, fail);
+                    }
+                    const int kn0 = min(nb, fail);
+                    GDoublePtr pa = opaque(A + j0 * lda + tid);
+                    auto store = [&](const double (&v)[16], int k0, int kn) {
+#pragma unroll
+                        for (int k = 0; k < 16; ++k) {
+                            if (tid < n && tid >= j0 + k0 + k && k0 + k < kn) *pa = v[k];
+                            pa += lda;
+                        }
+                    };
+                    store(a, 0, kn0);
+                    // row K's own entry of the left half holds l_kk: its right half is above the diagonal
+#pragma unroll
+                    for (int k = 0; k < 16; ++k) {
+                        b[k] = P[16 + k][tid];
+                        e[k] = P[16 + k][q1];
+                    }
+                    apply_columns<0>(e, b, d1, a);
+                    right_columns<0>(e, b, tid - j0, nb, fail);
+                    store(b, 16, min(nb, fail));
+                } else {
+                    double a[PW], d0[16], d1[PW];
+                    const int q0 = min(j0 + li, n - 1), q1 = min(j0 + 16 + li, n - 1);
+#pragma unroll
+                    for (int k = 0; k < PW; ++k) {
+                        a[k] = P[k][tid];
+                        d1[k] = P[k][q1];
+                        if (k < 16) d0[k] = P[k][q0];
+                    }
+                    panel_columns<0>(d0, d1, a, tid - j0, nb, fail);
+                    const int kn = min(nb, fail);
+                    GDoublePtr pa = opaque(A + j0 * lda + tid);
+#pragma unroll
+                    for (int k = 0; k < PW; ++k) {
+                        if (tid < n && tid >= j0 + k && k < kn) *pa = a[k];
+                        pa += lda;
+                    }
                 }
+                if (fail < PW) failed = fail;           // the same in every wavefront
             }
             __syncthreads();
             if (failed < PW) {
