@@ -182,7 +182,7 @@ struct Mixed {
     // the row exponents already in sm.cexp.  Sets sm.flag on a non-finite entry.
     static __device__ __forceinline__ void load_block(Smem &sm, const double *A, int lda, int n, int c0, int nb, bool chol)
     {
-        const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+        const int lane = opaque((int)threadIdx.x) & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         // LC columns per wavefront in flight at once (rows lane + 64 r)
         constexpr int LC = RPL <= 4 ? 4 : 2;
 #pragma unroll 1
@@ -245,14 +245,28 @@ struct Mixed {
     static __device__ __forceinline__ void apply_chunk(Smem &sm, int n, int c0, int kq, int kb, int cs, int ce, const float *Fg,
                                        int kl0, bool chol, int rlo)
     {
-        const int tid = threadIdx.x;
+        const int tid = opaque((int)threadIdx.x);
+        // The diagonal block first, then the product's L values, which stay in
+        // flight while U is formed (loads return in order).
+        float lv[RB][8];
+        constexpr int TPT = CH * CH / kT;
+        float dt[TPT];
         if (!chol) {
-            for (int e = tid; e < (2 * CH - 1) * CH; e += kT) {
-                const int i = e / CH, i2 = e % CH;      // row i (< 2 CH - 1), column i2
-                float v = 0.0f;
+#pragma unroll
+            for (int j = 0; j < TPT; ++j) {
+                const int e = tid + kT * j, i = e / CH, i2 = e % CH;     // row i, column i2
+                dt[j] = 0.0f;
                 if (i2 < i && i < kb)
-                    v = Fg ? Fg[mixed_diag_offset(n) + 32 * (size_t)kq + CH * i + i2] : sm.u.f.blk[kl0 + i2][sm.p[kq + i]];
-                sm.u.f.LT[i2][i] = v;
+                    dt[j] = Fg ? Fg[mixed_diag_offset(n) + 32 * (size_t)kq + e] : sm.u.f.blk[kl0 + i2][sm.p[kq + i]];
+            }
+        }
+        if (Fg) load_stored(n, kq, Fg, rlo, lv);
+        if (!chol) {
+#pragma unroll
+            for (int j = 0; j < TPT; ++j) {
+                const int e = tid + kT * j, i = e / CH, i2 = e % CH;
+                sm.u.f.LT[i2][i] = dt[j];
+                if (i < CH - 1) sm.u.f.LT[i2][CH + i] = 0.0f;
             }
             __syncthreads();
             // U of the chunk's pivot rows: eight threads per column, four rows
@@ -303,21 +317,18 @@ struct Mixed {
             }
         }
         __syncthreads();
-        gemm(sm, n, kq, kb, cs, ce, Fg, kl0, rlo);
+        if (Fg) gemm_stored(sm, n, kq, kb, cs, ce, rlo, lv);
+        else gemm(sm, n, kq, kb, cs, ce, kl0, rlo);
         __syncthreads();
     }
 
     // blk[c][o] -= sum_k L(o, kq+k) * U(k, c) for c in [cs, ce) and rows o >= rlo
     // with pivpos[o] >= kq + kb; -U^T is staged in Uh/Ul.
-    static __device__ __forceinline__ void gemm(Smem &sm, int n, int kq, int kb, int cs, int ce, const float *Fg, int kl0, int rlo)
+    static __device__ __forceinline__ void gemm(Smem &sm, int n, int kq, int kb, int cs, int ce, int kl0, int rlo)
     {
-        const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+        const int lane = opaque((int)threadIdx.x) & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         const int li = lane & 15, lk = lane >> 4;
         const int ostart = (rlo / 16) * 16;
-        if (Fg) {
-            gemm_stored(sm, n, kq, kb, cs, ce, Fg, rlo);
-            return;
-        }
 #pragma unroll 1
         for (int o0 = ostart + 16 * w; o0 < n; o0 += 16 * kWaves) {
             const int o = o0 + li;
@@ -329,7 +340,7 @@ struct Mixed {
                 for (int t = 0; t < 4; ++t) {
                     const int k = 16 * ks + 4 * lk + t;
                     float v = 0.0f;
-                    if (act && k < kb) v = Fg ? Fg[o + (size_t)(kq + k) * n] : sm.u.f.blk[kl0 + k][o];
+                    if (act && k < kb) v = sm.u.f.blk[kl0 + k][o];
                     _Float16 h, l;
                     split(v, h, l);
                     lh[ks][t] = h;
@@ -363,20 +374,17 @@ struct Mixed {
         }
     }
 
-    // The same product with L from the factor storage: every L value of the
-    // wavefront's row blocks is loaded first (one round of memory latency per
-    // chunk instead of one per row block), by buffer loads whose column part
-    // is a scalar offset.  Loads past column n - 1 (a partial last chunk) stay
-    // inside the factor storage and are discarded.
+    // L of the product below from the factor storage: every value of the
+    // wavefront's row blocks, by buffer loads whose column part is a scalar
+    // offset.  Loads past column n - 1 (a partial last chunk) stay inside the
+    // factor storage and are discarded.
     static constexpr int RB = NMAX / (16 * kWaves);     // row blocks per wavefront
-    static __device__ __forceinline__ void gemm_stored(Smem &sm, int n, int kq, int kb, int cs, int ce, const float *Fg,
-                                                       int rlo)
+    static __device__ __forceinline__ void load_stored(int n, int kq, const float *Fg, int rlo, float (&lv)[RB][8])
     {
-        const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+        const int lane = opaque((int)threadIdx.x) & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         const int li = lane & 15, lk = lane >> 4;
         const int ob = (rlo / 16) * 16 + 16 * w;
         const __amdgpu_buffer_rsrc_t Fr = rsrc(Fg, 4u * (unsigned)mixed_factor_floats(n));
-        float lv[RB][8];
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
             const int o = min(ob + 16 * kWaves * rb + li, n - 1);
@@ -388,6 +396,15 @@ struct Mixed {
                     lv[rb][4 * ks + t] =
                         __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(Fr, vo, 4 * n * (kq + 16 * ks + t), 0));
         }
+    }
+
+    // The same product with those L values.
+    static __device__ __forceinline__ void gemm_stored(Smem &sm, int n, int kq, int kb, int cs, int ce, int rlo,
+                                                       const float (&lv)[RB][8])
+    {
+        const int lane = opaque((int)threadIdx.x) & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        const int li = lane & 15, lk = lane >> 4;
+        const int ob = (rlo / 16) * 16 + 16 * w;
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
             const int o0 = ob + 16 * kWaves * rb;
@@ -438,7 +455,7 @@ struct Mixed {
     // Returns nonzero on a zero or NaN pivot.
     static __device__ __forceinline__ int panel_lu(Smem &sm, int n, int c0, int s0, int kb, int *ipiv)
     {
-        const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+        const int tid = opaque((int)threadIdx.x), lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
         float a[RPT][CH];
         int cur[RPT];
         bool act[RPT];
@@ -526,7 +543,7 @@ struct Mixed {
     // ---- Cholesky chunk panel: columns [s0, s0+kb) of the block, rows >= c0+s0 ----
     static __device__ __forceinline__ int panel_chol(Smem &sm, int n, int c0, int s0, int kb)
     {
-        const int tid = threadIdx.x;
+        const int tid = opaque((int)threadIdx.x);
         const int d0 = c0 + s0;          // first row / column of the diagonal block
         float a[RPT][CH];
         int bad = 0;
@@ -583,7 +600,7 @@ struct Mixed {
     // ---- block column to the factor storage ----------------------------------
     static __device__ __forceinline__ void write_block(Smem &sm, float *F, int n, int c0, int nb, bool chol)
     {
-        const int tid = threadIdx.x;
+        const int tid = opaque((int)threadIdx.x);
         if (!chol) {
             for (int e = tid; e < nb * n; e += kT) {
                 const int cc = e / n, o = e % n;
@@ -615,7 +632,7 @@ struct Mixed {
     // ---- the whole FP32 factorization; returns the status code --------------
     static __device__ __forceinline__ int factor(Smem &sm, const double *A, int lda, int n, float *F, int *ipiv, bool chol)
     {
-        const int tid = threadIdx.x;
+        const int tid = opaque((int)threadIdx.x);
         for (int o = tid; o < NMAX; o += kT) {
             sm.pivpos[o] = chol ? o : ((o < n) ? INT_MAX : -1);
             sm.p[o] = o;
@@ -679,7 +696,7 @@ struct Mixed {
     // pivot order and exponents of a stored factorization
     static __device__ __forceinline__ void load_factor_meta(Smem &sm, const float *F, int n, bool chol)
     {
-        const int tid = threadIdx.x;
+        const int tid = opaque((int)threadIdx.x);
         const int *Fexp = reinterpret_cast<const int *>(F + (size_t)n * n);
         for (int o = tid; o < n; o += kT) {
             sm.cexp[o] = Fexp[o];
@@ -698,12 +715,13 @@ struct Mixed {
     // next diagonal block while the columns are applied.  With each loaded where
     // it is used a step waited for memory twice: 83 us for both sweeps of a
     // matrix of order 256 among 768, 52 us this way (8192 systems 11.4 -> 10.4
-    // ms).  Prefetching a chunk's L the same way in apply_chunk spilled at three
-    // workgroups per CU and was slower (11.5 ms).
+    // ms).  Each phase takes the thread index through opaque(): addresses kept
+    // from phase to phase spilled 75 registers at three workgroups per CU (10.4
+    // -> 10.2 ms with the loads of apply_chunk, which need those registers).
     template <bool FWD>
     static __device__ __forceinline__ void sweep(Smem &sm, const float *F, int n, int nr, bool chol)
     {
-        const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+        const int tid = opaque((int)threadIdx.x), lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
         const int nch = (n + CH - 1) / CH;
         constexpr int TPT = CH * CH / kT;       // diagonal block entries per thread
         float t[TPT];
@@ -722,6 +740,7 @@ struct Mixed {
         load_diag(FWD ? 0 : (nch - 1) * CH);
 #pragma unroll 1
         for (int s = 0; s < nch; ++s) {
+            const int tid = opaque((int)threadIdx.x), lane = tid & 63;
             const int kq = CH * (FWD ? s : nch - 1 - s);
             const int kb = min(CH, n - kq);
 #pragma unroll
@@ -796,7 +815,7 @@ struct Mixed {
     static __device__ __forceinline__ int refine(Smem &sm, const double *A, int lda, const double *B, int ldb, double *X, int ldx,
                                  const float *F, int n, int nr, bool chol, double &anrm, double &berr)
     {
-        const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+        const int tid = opaque((int)threadIdx.x), lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
         const double eps = 0x1p-53;
         for (int e = tid; e < RG * NMAX; e += kT) {
             const int g = e / NMAX, o = e % NMAX;
