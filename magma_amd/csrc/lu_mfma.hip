@@ -179,6 +179,10 @@ __global__ void __launch_bounds__(MT) __attribute__((amdgpu_waves_per_eu(2))) ge
         const GDoublePtr A = (GDoublePtr)s.A[id];
         int *ipiv = s.ipiv[id];
         const int mn = min(m, n);
+        if (mn <= 0) {                              // no entries, and maybe no memory either
+            if (tid == 0) s.info[id] = 0;
+            continue;
+        }
         const int npan = (mn + PW - 1) / PW;        // factored chunks
         const int nblk = (n + PW - 1) / PW;
         int info = 0;

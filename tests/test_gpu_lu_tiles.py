@@ -64,3 +64,35 @@ def test_getrf_special(queue, oracle, n):
     assert np.array_equal(info.cpu().numpy(), info_o)
     assert np.array_equal(ipiv.numpy(), ipo)
     assert same(dA.numpy(), LUo)
+
+
+@pytest.mark.parametrize("nocheck", [False, True])
+def test_getrf_vbatched_empty(queue, oracle, nocheck):
+    """Matrices without rows or columns, with null pointers, in every size class
+    of the kernel beside ordinary ones: info 0, nothing read, the others as ever."""
+    import magma_amd as ma
+    rng = np.random.default_rng(11)
+    shapes = [(0, 100), (100, 0), (70, 66), (0, 200), (256, 0), (130, 129), (300, 0), (0, 512), (257, 40)]
+    V = ma.VarBatch([rng.uniform(-1, 1, (n, m)) for m, n in shapes])
+    for i, (m, n) in enumerate(shapes):
+        if m == 0 or n == 0:
+            V.ptrs[i] = 0
+    ipiv = ma.VarInts([max(1, min(s)) for s in shapes])
+    info = ma.dev_ints(np.full(len(shapes), -1))
+    print(f"getrf_vbatched with empty matrices nocheck={nocheck}", flush=True)
+    before = V.matrices()
+    L = ma.load()
+    if nocheck:
+        ret = L.magma_dgetrf_vbatched_max_nocheck(V.d_rows.data_ptr(), V.d_cols.data_ptr(), 512, V.ptr,
+                                                  V.d_ld.data_ptr(), ipiv.ptr, info.data_ptr(), V.count, queue.handle)
+        queue.sync()
+    else:
+        ret = L.magma_dgetrf_vbatched(V.d_rows.data_ptr(), V.d_cols.data_ptr(), V.ptr, V.d_ld.data_ptr(), ipiv.ptr,
+                                      info.data_ptr(), V.count, queue.handle)
+    assert ret == 0
+    assert info.cpu().numpy()[: V.count].tolist() == [0] * V.count
+    got = V.matrices()
+    for i, (m, n) in enumerate(shapes):
+        if m and n:
+            LUo, ipo, _ = oracle.dgetrf(before[i], m=m, n=n)
+            assert np.array_equal(ipiv.numpy(i, min(m, n)), ipo) and same(got[i], LUo), i
