@@ -27,6 +27,7 @@
 // callers test that and redo such a matrix with the reference loops.
 #pragma once
 
+#include "dpp_fma.h"
 #include "kernels.h"
 
 namespace magma_amd {
@@ -144,25 +145,52 @@ __device__ __forceinline__ void tri_sweep(TriView v, int n, double *X)
         return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, lane_off, off, 0));
     };
     auto at = [&](int t) { return 16 * (rev ? nt - 1 - t : t); };           // first matrix row of block t
-    auto xrow = [&](int s) { return (rev ? 16 * nt - 1 - s : s) * kTriPitch + li; };
+    auto xrow = [&](int s, int li) { return (rev ? 16 * nt - 1 - s : s) * kTriPitch + li; };
+    // Block eb (-1: none) holds the matrix's last rows and rows past n.  Its tiles
+    // repeat row and column n - 1 there, so that every load stays inside the
+    // matrix (the resource's range check does not cover the scalar offset); what
+    // the repeats bring is cleared or masked where it is used.
+    const int last = n - 1 - 16 * (nt - 1), eb = last == 15 ? -1 : rev ? 0 : nt - 1;
+    const int tile_e = min(li, last) * ds + lk * dk;        // rows of eb, forward
     // factor tile below the diagonal: A operand of slice i, entry (row li, column 4 i + lk)
     auto load_tile = [&](int tr, int tc, d4 &a) {
+        const int lane_off = tr == eb ? tile_e : tile;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) a[i] = ld(tile, at(tr) * ds + (at(tc) + 4 * (rev ? 3 - i : i)) * dk);
+        for (int i = 0; i < 4; ++i) a[i] = ld(lane_off, at(tr) * ds + (at(tc) + 4 * (rev ? 3 - i : i)) * dk);
+    };
+    // the same where the tile's columns are those of eb
+    auto load_edge = [&](int tr, d4 &a) {
+        const int l = opaque(lane);
+        const int r = rev ? 15 - (l & 15) : l & 15, k = rev ? 15 - (l >> 4) : l >> 4;
+        const int row = (tr == eb ? min(r, last) : r) * ds;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            a[i] = ld(row + min(rev ? k - 4 * i : k + 4 * i, last) * dk, at(tr) * ds + at(eb) * dk);
+    };
+    auto load_diag = [&](int t, d4 &a) {
+        if (t == eb) load_edge(t, a);
+        else load_tile(t, t, a);
     };
     d4 x[NB], av[NB], dt;
-    load_tile(min(w, nt - 1), min(w, nt - 1), dt);
+    load_diag(min(w, nt - 1), dt);
+    // With one wavefront the LDS addresses are formed where they are used: kept
+    // from block to block they spilled up to 25 of the 128 registers (20,000 of
+    // order 64: getri 818 -> 776 us, trsm with 16 vectors 256 -> 252 us).
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
+        const int ln = W == 1 ? opaque(lane) : lane, li = ln & 15, lk = ln >> 4;
         const int t = w + W * b;
         x[b] = d4{0.0, 0.0, 0.0, 0.0};
         av[b] = x[b];
         if (t < nt) {
-            if (t > 0) load_tile(t, 0, av[b]);
+            if (t > 0) {
+                if (eb == 0) load_edge(t, av[b]);
+                else load_tile(t, 0, av[b]);
+            }
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int s = 16 * t + 4 * i + lk;
-                if (rev ? s >= pad : s < n) x[b][i] = X[xrow(s)];
+                if (rev ? s >= pad : s < n) x[b][i] = X[xrow(s, li)];
             }
         }
     }
@@ -184,8 +212,9 @@ __device__ __forceinline__ void tri_sweep(TriView v, int n, double *X)
         for (int ww = 0; ww < W; ++ww) {
             const int t = t0 + ww;
             if (t >= nt) break;
-            if (W == 1 || w == ww) {
-                if (!rev && 16 * t + 16 > n) {
+            const int ln = W == 1 ? opaque(lane) : lane, li = ln & 15, lk = ln >> 4;
+                if (W == 1 || w == ww) {
+                if (!rev && t == eb) {
                     // rows past n come last: the same there
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
@@ -197,9 +226,9 @@ __device__ __forceinline__ void tri_sweep(TriView v, int n, double *X)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int s = 16 * t + 4 * i + lk;
-                    if (rev ? s >= pad : s < n) X[xrow(s)] = x[0][i];
+                    if (rev ? s >= pad : s < n) X[xrow(s, li)] = x[0][i];
                 }
-                if (t + W < nt) load_tile(t + W, t + W, dt);
+                if (t + W < nt) load_diag(t + W, dt);
             }
             if (t + 1 >= nt) break;
             d4 xb;
@@ -210,7 +239,7 @@ __device__ __forceinline__ void tri_sweep(TriView v, int n, double *X)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int s = 16 * t + 4 * i + lk;
-                    xb[i] = s >= pad ? -X[xrow(s)] : 0.0;
+                    xb[i] = s >= pad ? -X[xrow(s, li)] : 0.0;
                 }
             }
 #pragma unroll

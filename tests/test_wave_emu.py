@@ -12,7 +12,7 @@ EMU = os.path.join(ROOT, "tests", "wave_emu")
 CSRC = os.path.join(ROOT, "magma_amd", "csrc")
 
 
-def _run(tmp_path, name):
+def _run(tmp_path, name, *args):
     clang = shutil.which("clang++", path="/opt/rocm/llvm/bin" + os.pathsep + os.environ.get("PATH", ""))
     if clang is None:
         pytest.skip("no clang++")
@@ -28,9 +28,13 @@ def _run(tmp_path, name):
     subprocess.run([clang, "-std=c++20", "-O1", "-march=native", "-ffp-contract=off", "-w", "-I" + str(tmp_path),
                     "-I" + EMU, "-I" + os.path.join(ROOT, "include"), os.path.join(EMU, name + ".cpp"), "-o", exe],
                    check=True)
-    r = subprocess.run([exe], capture_output=True, text=True, timeout=300)
+    r = subprocess.run([exe, *args], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and r.stdout.strip().endswith("ok"), (r.returncode, r.stdout[-2000:] + r.stderr[-2000:])
 
 
 def test_lu_of_empty_matrices(tmp_path):
     _run(tmp_path, "lu")
+
+
+def test_sweeps_load_inside_the_matrix(tmp_path):
+    _run(tmp_path, "sweeps", "loads")
