@@ -213,14 +213,23 @@ __device__ __forceinline__ void tri_sweep(TriView v, int n, double *X)
             const int t = t0 + ww;
             if (t >= nt) break;
             const int ln = W == 1 ? opaque(lane) : lane, li = ln & 15, lk = ln >> 4;
-                if (W == 1 || w == ww) {
-                if (!rev && t == eb) {
-                    // rows past n come last: the same there
+            if (W == 1 || w == ww) {
+                // Rows past n come last in a forward sweep: no coupling and a unit
+                // diagonal there too, and zeros in x, since what the updates left
+                // would reach the rows above through the block's MFMAs if it is
+                // not finite (0 times Inf).
+                const bool edge = !rev && t == eb;
+                if (edge) {
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const int k = 4 * i + lk;
                         if (16 * t + max(k, li) >= n) dt[i] = k == li ? 1.0 : 0.0;
                     }
+                }
+                if (W == 1 || edge) {           // in a branch it costs one wavefront spills
+                    const int lim = rev ? 16 * nt : n;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) x[0][i] = 16 * t + 4 * i + lk < lim ? x[0][i] : 0.0;
                 }
                 diag_solve<DIAG>(x[0], dt, li, lk);
 #pragma unroll

@@ -164,3 +164,37 @@ def test_getri_tiles(queue, oracle, n):
     for s in range(2):
         assert same(dI.numpy()[s], oracle.dgetrs(LU[s], ipiv[s], np.eye(n))), s
     assert info.cpu().tolist() == [0, n // 2 + 1]
+
+
+@pytest.mark.parametrize("n", [17, 27, 64, 65, 129, 257, 491])
+def test_unread_values_do_not_leave_the_sweeps(queue, n):
+    """With NaN in the padding and in the triangle that is not read, the solves
+    stay with the register sweeps.  Only those turn zeros of a zero right-hand
+    side over a negative diagonal into -0 (back, after potrs's second sweep): the reference loops, which
+    a result that is not finite goes back to, skip a zero and keep its sign."""
+    import magma_amd as ma
+    import torch
+    rng = np.random.default_rng(n)
+    F, _ = factor_batch(rng, 2, n)
+    F[:, np.arange(n), np.arange(n)] = -np.abs(F[:, np.arange(n), np.arange(n)])
+    low = np.where(np.tril(np.ones((n, n), bool)).T, F, np.nan)        # storage is transposed
+    B = rng.uniform(-1, 1, (2, 5, n))
+    B[:, 2] = 0.0
+    L = ma.load()
+    for ld in (n, n + 3):
+        print(f"sweeps n={n} ld={ld}", flush=True)
+        dA, dB = device(low, ld), device(B, n)
+        L.magmablas_dtrsm_batched(ma.MagmaLeft, ma.MagmaLower, ma.MagmaNoTrans, ma.MagmaNonUnit, n, 5, 1.0, dA.ptr,
+                                  dA.ld, dB.ptr, dB.ld, 2, queue.handle)
+        X = dB.numpy()
+        assert np.isfinite(X).all() and (X[:, 2] == 0).all() and np.signbit(X[:, 2]).any(axis=1).all()
+        dB = device(B, n)
+        assert ma.dpotrs_batched(dA, dB, queue, uplo=ma.MagmaLower) == 0
+        X = dB.numpy()
+        assert np.isfinite(X).all() and (X[:, 2] == 0).all() and not np.signbit(X[:, 2, n - 1]).any()
+        dA, dB = device(F, ld), device(B, n)
+        ip = ma.IntBatch(2, n)
+        ip.t.copy_(torch.arange(1, n + 1, dtype=torch.int32).repeat(2, 1))
+        assert ma.dgetrs_batched(dA, ip, dB, queue) == 0
+        X = dB.numpy()
+        assert np.isfinite(X).all() and (X[:, 2] == 0).all() and np.signbit(X[:, 2]).any(axis=1).all()

@@ -38,3 +38,7 @@ def test_lu_of_empty_matrices(tmp_path):
 
 def test_sweeps_load_inside_the_matrix(tmp_path):
     _run(tmp_path, "sweeps", "loads")
+
+
+def test_sweeps_keep_out_what_is_not_read(tmp_path):
+    _run(tmp_path, "sweeps", "values")

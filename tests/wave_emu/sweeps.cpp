@@ -1,7 +1,8 @@
 // tri_sweep of every direction, triangle and scaling against plain loops, the
 // operand ending at a page that must not be touched: its loads stay inside the
-// matrix ("loads"), and nothing that a solve does not read (the other triangle,
-// the padding of lda; all NaN here) reaches a result ("values").
+// matrix ("loads"), and neither what a solve does not read (the other triangle,
+// the padding of lda; all NaN here) nor the rows past n that fill the last block
+// reach a result ("values").
 #include <hip/hip_runtime.h>
 
 #include "tri_mfma.h"
@@ -13,7 +14,7 @@ static double uniform(double lo, double hi) { return lo + (hi - lo) * (rand() / 
 static bool values;
 
 template <int W, int NB, TriDiag DIAG>
-static bool one(int n, int lda, bool lower, bool trans)
+static bool one(int n, int lda, bool lower, bool trans, bool large = false)
 {
     const size_t elems = (size_t)(n - 1) * lda + n;
     double *a = emu::guard(elems, false), *X = emu::guard((size_t)n * kTriPitch, false);
@@ -25,6 +26,13 @@ static bool one(int n, int lda, bool lower, bool trans)
     }
     for (int r = 0; r < n; ++r)
         for (int c = 0; c < 16; ++c) X[r * kTriPitch + c] = want[r * 16 + c] = c == 3 ? 0.0 : uniform(-1, 1);
+    if (large) {
+        // unit lower: the last row's sum is in range, but not without its start
+        for (int i = 1; i < n; ++i) a[i] = i == n - 1;
+        for (int i = 2; i < n; ++i) a[i + (size_t)lda] = i == n - 1;
+        for (int c = 0; c < 16; ++c)
+            for (int r : {0, 1, n - 1}) X[r * kTriPitch + c] = want[r * 16 + c] = r == n - 1 ? 1.6e308 : 1e308;
+    }
     const bool forward = lower != trans;
     for (int s = 0; s < n; ++s) {
         const int k = forward ? s : n - 1 - s;
@@ -62,6 +70,7 @@ static bool all(std::initializer_list<int> orders)
             const bool lower = v & 1, trans = v & 2;
             ok &= one<W, NB, kTriDivide>(n, n, lower, trans);
             ok &= one<W, NB, kTriUnit>(n, n + 3, lower, trans);
+            if (n > 2 && lower && !trans) ok &= one<W, NB, kTriUnit>(n, n, lower, trans, true);
             if (n % 16 == 1) ok &= one<W, NB, kTriReciprocal>(n, n + 1, lower, trans);
         }
     return ok;
