@@ -428,7 +428,11 @@ __global__ void __launch_bounds__(256) geqrf_kernel(int m, int n, double **A_arr
             // max |x| and sum (x / max)^2: wavefront shuffles, then the four
             // wavefronts' values through LDS
             double mx = 0.0;
-            for (int r = i + 1 + tid; r < m; r += 256) mx = fmax(mx, fabs(AQ(r, i)));
+            // a NaN, which fmax would drop, counts as Inf: the scaled sum is then NaN
+            for (int r = i + 1 + tid; r < m; r += 256) {
+                const double x = fabs(AQ(r, i));
+                mx = fmax(mx, x == x ? x : __builtin_huge_val());
+            }
             for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off));
             if (lane == 0) redm[wave] = mx;
             __syncthreads();
@@ -448,7 +452,8 @@ __global__ void __launch_bounds__(256) geqrf_kernel(int m, int n, double **A_arr
                 double t = 0.0, beta = alpha, sc = 0.0;
                 if (xnorm != 0.0) {
                     const double xa = fabs(alpha), wmax = fmax(xa, xnorm), wmin = fmin(xa, xnorm);
-                    const double hyp = wmax * sqrt(1.0 + (wmin / wmax) * (wmin / wmax));
+                    const double hyp = (xa == xa && xnorm == xnorm)
+                                           ? wmax * sqrt(1.0 + (wmin / wmax) * (wmin / wmax)) : xa + xnorm;
                     beta = -copysign(hyp, alpha);
                     t = (beta - alpha) / beta;
                     sc = 1.0 / (alpha - beta);

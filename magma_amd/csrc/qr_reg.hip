@@ -93,11 +93,13 @@ __global__ void __launch_bounds__(64 * W, 2) geqrf_reg_kernel(int m, int n, doub
     __shared__ double2 vbuf[2][MT / 2 + 1];      // the reflector; then tau
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int g = lane % RG, cpos = wave * CG + lane / RG;
-    const int k = min(m, n);
+    // The last row has no reflector (rows past m may hold NaN by then).
+    const int k = min(m - 1, n);
     for (int id = blockIdx.x; id < count; id += gridDim.x) {
         GDoublePtr A = (GDoublePtr)A_array[id];
         GDoublePtr tau = (GDoublePtr)tau_array[id];
         if (tid == 0 && info) info[id] = 0;
+        if (tid == 0 && m <= n) tau[m - 1] = 0.0;
         double a[CL][RL];
 #pragma unroll
         for (int c = 0; c < CL; ++c)
@@ -159,7 +161,8 @@ __global__ void __launch_bounds__(64 * W, 2) geqrf_reg_kernel(int m, int n, doub
                                 sq = fma(y, y, sq);
                             }
                         }
-                        const double xnorm = amax * sqrt(lane_value(group_sum<RG>(sq), owner));
+                        // fmax drops a NaN: where it is all the column has, amax is 0
+                        const double xnorm = ss == ss ? amax * sqrt(lane_value(group_sum<RG>(sq), owner)) : ss;
                         if (xnorm != 0.0) {
                             const double xa = fabs(alpha), wmax = fmax(xa, xnorm), wmin = fmin(xa, xnorm);
                             // fmax and fmin would drop a NaN

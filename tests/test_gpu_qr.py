@@ -61,3 +61,22 @@ def test_nonfinite_stays_in_its_columns(queue, oracle, m, n):
     _, Fr, Tr = run(queue, np.where(np.isfinite(A), A, 0.5), m)
     assert np.array_equal(F[0][: n - 1], Fr[0][: n - 1]) and np.array_equal(T[0][: n - 1], Tr[0][: n - 1])
     assert np.isnan(oracle.dgeqrf(A[1])[1][0]) and np.isnan(T[1][0])
+
+
+@pytest.mark.parametrize("m,n", [(2, 2), (40, 40), (65, 33), (100, 100), (128, 7), (129, 129), (300, 3)])
+def test_a_lone_nan_reaches_tau(queue, oracle, m, n):
+    """A NaN that is all a column has below its diagonal, in the first column
+    (matrix 0) and in the last one that has a reflector (1): tau and R are NaN
+    exactly where dgeqr2's are."""
+    rng = np.random.default_rng(m + n)
+    k = min(m - 1, n) - 1
+    A = np.stack([np.triu(rng.uniform(1, 2, (m, n))).T] * 2)        # storage is transposed
+    A[0][0, m - 1] = np.nan
+    A[1][k, k + 1] = np.nan
+    print(f"geqrf nan m={m} n={n}", flush=True)
+    _, F, T = run(queue, A, m)
+    for s, i in enumerate((0, k)):
+        Fo, to = oracle.dgeqrf(A[s])
+        assert np.isnan(to[i]) and np.array_equal(np.isnan(T[s]), np.isnan(to)), s
+        top = np.triu(np.ones((m, n), bool)).T
+        assert np.array_equal(np.isnan(F[s][top]), np.isnan(Fo[top])), s
