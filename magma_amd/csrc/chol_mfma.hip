@@ -65,7 +65,6 @@ __device__ __forceinline__ void panel_columns(double (&d0)[16], double (&d1)[PW]
         }
         const double l = rc * a[K];
         a[K] = row == K ? ljj : l;
-        dpp_operand(x0, x1);
         if constexpr (K < 16) fmac_row<K + 1, 16>(d0, x0, x1, d0[K]);
         fmac_row<K + 1, PW>(d1, x0, x1, d1[K]);
         fmac_row<K + 1, PW>(a, x0, x1, l);
@@ -85,10 +84,9 @@ __device__ __forceinline__ void left_columns(double (&d0)[16], double (&d1)[16],
         const double ljj = sqrt(dkk), rc = 1.0 / ljj;
         d0[K] = rc * d0[K];
         d1[K] = rc * d1[K];
-        double x0 = -d0[K], x1 = x0;
+        const double x0 = -d0[K];
         const double l = rc * a[K];
         a[K] = row == K ? ljj : l;
-        dpp_operand(x0, x1);
         fmac_row<K + 1, 16>(d0, x0, x0, d0[K]);
         fmac_row<K + 1, 16>(d1, x0, x0, d1[K]);
         fmac_row<K + 1, 16>(a, x0, x0, l);
@@ -103,8 +101,7 @@ __device__ __forceinline__ void apply_columns(double (&e)[16], double (&b)[16], 
                                               const double (&a)[16])
 {
     if constexpr (K < 16) {
-        double x = -d1[K], y = x;
-        dpp_operand(x, y);
+        const double x = -d1[K];
         fmac_row<0, 16>(e, x, x, d1[K]);
         fmac_row<0, 16>(b, x, x, a[K]);
         apply_columns<K + 1>(e, b, d1, a);
@@ -120,10 +117,9 @@ __device__ __forceinline__ void right_columns(double (&e)[16], double (&b)[16], 
         if (16 + K < nb && !(dkk > 0.0)) fail = min(fail, 16 + K);
         const double ljj = sqrt(dkk), rc = 1.0 / ljj;
         e[K] = rc * e[K];
-        double x = -e[K], y = x;
+        const double x = -e[K];
         const double l = rc * b[K];
         b[K] = row == 16 + K ? ljj : l;
-        dpp_operand(x, y);
         fmac_row<K + 1, 16>(e, x, x, e[K]);
         fmac_row<K + 1, 16>(b, x, x, l);
         right_columns<K + 1>(e, b, row, nb, fail);

@@ -12,6 +12,8 @@ namespace magma_amd {
 typedef double __attribute__((address_space(1))) *GDoublePtr;
 typedef float __attribute__((address_space(1))) *GFloatPtr;
 typedef int __attribute__((address_space(1))) *GIntPtr;
+// and in LDS
+typedef double __attribute__((address_space(3))) *LDoublePtr;
 
 // Describes a set of matrices for one launch.  Sizes either fixed (arrays
 // null) or per matrix (device arrays indexed by matrix id).  `index`, when not

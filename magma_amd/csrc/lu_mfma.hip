@@ -67,6 +67,9 @@ constexpr int PW = 32;              // columns of a block column
 constexpr int GW = 16;              // columns of a panel group
 constexpr int TPW = 4;              // 16-row tiles per wavefront
 
+typedef double d2 __attribute__((ext_vector_type(2)));
+typedef d2 __attribute__((address_space(3))) *LDouble2Ptr;
+
 __device__ __forceinline__ int pick(const int *arr, int fixed, int id) { return arr ? arr[id] : fixed; }
 
 template <int MT>
@@ -364,6 +367,7 @@ __global__ void __launch_bounds__(MT) __attribute__((amdgpu_waves_per_eu(2))) ge
 #pragma unroll
             for (int k = 0; k < PW; ++k) a[k] = sm.P[k][tid];
             if (p + 1 < nblk) load_c(j0 + PW);
+            tid = opaque(tid);
             const int pos0 = pos, info0 = info;
             double z = 0.0;                         // NaN when an entry of this row is not finite
             // GW columns at a time; the rest of the row then moves down to the
@@ -383,17 +387,21 @@ __global__ void __launch_bounds__(MT) __attribute__((amdgpu_waves_per_eu(2))) ge
                     const long long av = __double_as_longlong(fabs(v));
                     int pp, pr;
                     select_pivot<W>(sm.slot, int4{(int)av, cand ? (int)(av >> 32) + 1 : 0, pos, tid}, w, pp, pr);
+                    // Above 128 rows the array lies past what an offset from 0
+                    // reaches, and 18 addresses were kept in registers: one address
+                    // and offsets (256 of order 500, 7 rhs: 2.45 -> 2.42 ms).
+                    constexpr bool far = offsetof(LuSmem<MT>, row) + sizeof(double) * (PW + 2) > 65536;
+                    const LDoublePtr row = far ? opaque((LDoublePtr)sm.row) : (LDoublePtr)sm.row;
                     if (tid == pr) {
-                        double2 *dst = reinterpret_cast<double2 *>(sm.row);
 #pragma unroll
-                        for (int k = jj & ~1; k < PW; k += 2) dst[k / 2] = make_double2(a[k], a[k + 1]);
-                        sm.row[PW] = rv;
+                        for (int k = jj & ~1; k < PW; k += 2) *(LDouble2Ptr)(row + k) = d2{a[k], a[k + 1]};
+                        row[PW] = rv;
                         sm.swaps[g + jj] = pp;
                     }
                     __syncthreads();
-                    const double piv = sm.row[jj], rc = sm.row[PW];
-                    double nu0 = -sm.row[tid & 15], nu1 = -sm.row[16 + (tid & 15)];
-                    dpp_operand(nu0, nu1);
+                    const double piv = row[jj], rc = row[PW];
+                    double nu0 = -row[tid & 15], nu1 = -row[16 + (tid & 15)];
+                    asm volatile("" : "+v"(nu0), "+v"(nu1));     // both reads here, not one in the branch below
                     if (piv == 0.0 && info == 0) info = j + 1;
                     bad |= piv != 0.0 && !(fabs(piv) >= DBL_MIN);
                     pos = (pos == j) ? pp : ((pos == pp) ? j : pos);

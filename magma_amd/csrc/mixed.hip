@@ -513,8 +513,7 @@ struct Mixed {
             }
             __syncthreads();
             const float piv = sm.row[jj], rc = sm.row[CH];
-            float nu0 = -sm.row[tid & 15], nu1 = -sm.row[16 + (tid & 15)];
-            dpp_operand(nu0, nu1);
+            const float nu0 = -sm.row[tid & 15], nu1 = -sm.row[16 + (tid & 15)];
             if (!(piv != 0.0f) || piv != piv) bad = 1;
 #pragma unroll
             for (int r = 0; r < RPT; ++r) {

@@ -18,12 +18,8 @@ inline void fmac_row(T (&a)[N], T x0, T x1, T l)
     }
 }
 
-template <class T>
-inline void dpp_operand(T &, T &)
-{
-}
-
 inline GDoublePtr opaque(GDoublePtr p) { return p; }
+inline LDoublePtr opaque(LDoublePtr p) { return p; }
 inline int opaque(int x) { return x; }
 
 }  // namespace magma_amd
