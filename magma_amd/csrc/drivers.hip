@@ -5,8 +5,9 @@
 // Dispatch (replaces the static crossover tables of
 // control/get_batched_crossover.cpp:25-228 and control/batched_kernel_param.h):
 //   max(m,n) <= 64   register-resident kernels, 64/NMAX matrices per wavefront
-//   max(m,n) <= 512  LU: workgroup per matrix, FP64 MFMA trailing update
-//   otherwise        blocked workgroup-per-matrix kernels (VALU)
+//   max(m,n) <= 512  LU: workgroup per matrix, FP64 MFMA updates
+//   otherwise, and where a side is at most 16 (see launch_getrf)
+//                    blocked workgroup-per-matrix kernels (VALU)
 #include <algorithm>
 
 #include "kernels.h"
@@ -16,7 +17,7 @@ namespace magma_amd {
 magma_int_t launch_getrf_small(const MatSet &s, int max_mn_dim, bool solve, hipStream_t st);
 magma_int_t launch_potrf_small(const MatSet &s, int max_n, bool solve, hipStream_t st);
 magma_int_t launch_getrf_blocked(const MatSet &s, int max_m, hipStream_t st);
-magma_int_t launch_getrf_mfma(const MatSet &s, int max_dim, hipStream_t st);
+magma_int_t launch_getrf_mfma(const MatSet &s, int max_dim, int max_m, hipStream_t st);
 magma_int_t launch_potrf_blocked(const MatSet &s, int max_n, hipStream_t st);
 
 constexpr int kRegMax = 64;
@@ -43,7 +44,14 @@ magma_int_t launch_getrf(const MatSet &s, int max_m, int max_n, bool fused_solve
 {
     const int dim = std::max(max_m, max_n);
     if (dim <= kRegMax) return launch_getrf_small(s, dim, fused_solve, st);
-    magma_int_t r = (dim <= kMfmaMax) ? launch_getrf_mfma(s, dim, st) : launch_getrf_blocked(s, max_m, st);
+    // A side of at most 16 leaves the MFMA kernel's block column half empty and,
+    // above 128 rows, its LDS holds one or two workgroups per CU: the VALU kernel
+    // (MFMA -> VALU, us: 8 x 512 x 4882 1094 -> 262, 16 x 128 x 8000 515 -> 351,
+    // 300 x 16 x 4166 374 -> 213; but 128 x 16 x 8000 222 -> 262, 512 x 32 x 1220
+    // 221 -> 336, 32 x 512 x 1220 440 -> 623).
+    const bool narrow = std::min(max_m, max_n) <= 16 && (max_m <= 16 || max_m > 128);
+    magma_int_t r = (dim <= kMfmaMax && !narrow) ? launch_getrf_mfma(s, dim, max_m, st)
+                                                 : launch_getrf_blocked(s, max_m, st);
     if (r != MAGMA_SUCCESS || !fused_solve) return r;
     return launch_getrs(s, 'N', max_n, 0, st);
 }

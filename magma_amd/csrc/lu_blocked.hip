@@ -1,5 +1,6 @@
 // lu_blocked.hip -- blocked right-looking LU and Cholesky, one 256-thread
-// workgroup per matrix, for orders above 512.
+// workgroup per matrix, for orders above 512 (and LU where one side is at most
+// 16).
 //
 // Per panel of PW columns:
 //   panel    the whole workgroup factors rows j0..m-1 x PW columns held in

@@ -490,14 +490,17 @@ static magma_int_t launch_mt(const MatSet &s, int variant, hipStream_t st)
     return MAGMA_SUCCESS;
 }
 
-// 64 < max(m, n) <= 512; returns MAGMA_ERR_NOT_SUPPORTED above.
-magma_int_t launch_getrf_mfma(const MatSet &s, int max_dim, hipStream_t st)
+// 64 < max_dim <= 512 (the largest m or n); returns MAGMA_ERR_NOT_SUPPORTED
+// above.  The kernel goes by the rows, which are what a workgroup's threads and
+// LDS hold; by the larger side, wide matrices left most of both idle (us:
+// 100 x 512 x 390 1003 -> 595, 64 x 300 x 1041 981 -> 426).
+magma_int_t launch_getrf_mfma(const MatSet &s, int max_dim, int max_m, hipStream_t st)
 {
     if (s.count <= 0) return MAGMA_SUCCESS;
     if (max_dim > 512) return MAGMA_ERR_NOT_SUPPORTED;
     const int v = tuned_variant(kTuneGetrf, size_class_of(max_dim));
-    if (max_dim <= 128) return launch_mt<128>(s, v, st);
-    if (max_dim <= 256) return launch_mt<256>(s, v, st);
+    if (max_m <= 128) return launch_mt<128>(s, v, st);
+    if (max_m <= 256) return launch_mt<256>(s, v, st);
     return launch_mt<512>(s, v, st);
 }
 

@@ -54,7 +54,7 @@ namespace magma_amd {
 
 magma_int_t launch_getrf_small_v(const MatSet &s, int max_mn_dim, bool solve, bool var, hipStream_t st);
 magma_int_t launch_potrf_small_v(const MatSet &s, int max_n, bool solve, bool var, hipStream_t st);
-magma_int_t launch_getrf_mfma(const MatSet &s, int max_dim, hipStream_t st);
+magma_int_t launch_getrf_mfma(const MatSet &s, int max_dim, int max_m, hipStream_t st);
 magma_int_t launch_getrf_blocked(const MatSet &s, int max_m, hipStream_t st);
 magma_int_t launch_potrf_blocked(const MatSet &s, int max_n, hipStream_t st);
 magma_int_t zero_info(int *info, int count, hipStream_t st);
@@ -1154,7 +1154,7 @@ magma_int_t launch_mixed_fallback(const MixedSet &g, int max_n, int max_nrhs, hi
             if (max_n <= 64) {
                 r = launch_getrf_small_v(s, max_n, true, var, st);
             } else {
-                r = (max_n <= 512) ? launch_getrf_mfma(s, max_n, st) : launch_getrf_blocked(s, max_n, st);
+                r = (max_n <= 512) ? launch_getrf_mfma(s, max_n, max_n, st) : launch_getrf_blocked(s, max_n, st);
                 if (r == MAGMA_SUCCESS) r = launch_getrs(s, 'N', max_n, 0, st);
             }
         } else {

@@ -38,7 +38,7 @@ namespace magma_amd {
 magma_int_t launch_getrf_small_v(const MatSet &s, int max_mn_dim, bool solve, bool var, hipStream_t st);
 magma_int_t launch_potrf_small_v(const MatSet &s, int max_n, bool solve, bool var, hipStream_t st);
 magma_int_t launch_getrf_blocked(const MatSet &s, int max_m, hipStream_t st);
-magma_int_t launch_getrf_mfma(const MatSet &s, int max_dim, hipStream_t st);
+magma_int_t launch_getrf_mfma(const MatSet &s, int max_dim, int max_m, hipStream_t st);
 magma_int_t launch_potrf_blocked(const MatSet &s, int max_n, hipStream_t st);
 magma_int_t launch_gemm_tiles(const GemmSet &g, const int *prefix, long max_tiles, int tile, hipStream_t st);
 magma_int_t zero_info(int *info, int count, hipStream_t st);
@@ -156,7 +156,7 @@ magma_int_t launch_class(char kind, int b, MatSet s, hipStream_t st)
     switch (kind) {
     case 'L':
         if (lim <= 64) return launch_getrf_small_v(s, lim, false, true, st);
-        return lim <= 512 ? launch_getrf_mfma(s, lim, st) : launch_getrf_blocked(s, lim, st);
+        return lim <= 512 ? launch_getrf_mfma(s, lim, lim, st) : launch_getrf_blocked(s, lim, st);
     case 'C': return lim <= 64 ? launch_potrf_small_v(s, lim, false, true, st) : launch_potrf_blocked(s, lim, st);
     case 'N':
     case 'T': return launch_getrs(s, kind, lim, 0, st);

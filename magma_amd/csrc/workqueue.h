@@ -7,7 +7,8 @@ namespace magma_amd {
 
 // Size classes by max(m, n): <=8, <=16, <=32, <=64, <=128, <=256, <=512,
 // <=1024, <=2048, <=8192 (the largest order the factor kernels take; callers
-// reject larger ones before binning).
+// reject larger ones before binning).  Of those above 64 and up to 512 by the
+// rows alone, as the LU kernels there are chosen (lu_mfma.hip): n may be larger.
 constexpr int kNumBuckets = 10;
 constexpr int kBucketLimit[kNumBuckets] = {8, 16, 32, 64, 128, 256, 512, 1024, 2048, 8192};
 

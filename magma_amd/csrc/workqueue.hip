@@ -17,10 +17,11 @@ namespace {
 
 constexpr int kScanThreads = 1024;
 
-// size class of an order-n matrix (see workqueue.h)
+// size class of an m x n matrix (see workqueue.h)
 __device__ __forceinline__ int size_class(int m, int n)
 {
-    const int d = max(m, n);
+    int d = max(m, n);
+    if (d > 64 && d <= 512) d = max(m, 65);
     if (d <= 8) return 0;
     if (d <= 16) return 1;
     if (d <= 32) return 2;

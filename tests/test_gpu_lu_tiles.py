@@ -96,3 +96,51 @@ def test_getrf_vbatched_empty(queue, oracle, nocheck):
         if m and n:
             LUo, ipo, _ = oracle.dgetrf(before[i], m=m, n=n)
             assert np.array_equal(ipiv.numpy(i, min(m, n)), ipo) and same(got[i], LUo), i
+
+
+# either side of the lines between the kernels: rows 128 / 256, a side of 16
+NARROW = [(8, 65), (65, 8), (16, 100), (17, 100), (16, 512), (17, 512), (128, 16), (129, 16), (129, 17), (300, 16),
+          (300, 17), (512, 1), (1, 512), (100, 512), (128, 400), (129, 400), (64, 300)]
+
+
+@pytest.mark.parametrize("m,n", NARROW)
+def test_getrf_wide_and_narrow(queue, oracle, m, n):
+    import magma_amd as ma
+    rng = np.random.default_rng(1000 * m + n)
+    A = rng.uniform(-1, 1, (3, n, m))
+    A[2] = rng.integers(-2, 3, size=(n, m))          # ties
+    print(f"getrf m={m} n={n}", flush=True)
+    dA = ma.DeviceBatch(A, ld=m + 1)
+    ret, ipiv, info = ma.dgetrf_batched(dA, queue, m=m, n=n)
+    assert ret == 0
+    got, ip, inf = dA.numpy(), ipiv.numpy(), info.cpu().numpy()
+    for s in range(3):
+        LUo, ipo, info_o = oracle.dgetrf(A[s], m=m, n=n)
+        assert inf[s] == info_o and np.array_equal(ip[s], ipo) and same(got[s], LUo), s
+
+
+@pytest.mark.parametrize("nocheck", [False, True])
+def test_getrf_vbatched_wide_and_narrow(queue, oracle, nocheck):
+    """The same shapes in one variable-size call, where wide matrices go by their rows."""
+    import magma_amd as ma
+    rng = np.random.default_rng(12)
+    shapes = NARROW + [(70, 600), (600, 70), (64, 64), (60, 65)]
+    mats = [rng.uniform(-1, 1, (n, m)) for m, n in shapes]
+    V = ma.VarBatch(mats)
+    ipiv = ma.VarInts([min(s) for s in shapes])
+    info = ma.dev_ints(np.full(len(shapes), -1))
+    print(f"getrf_vbatched wide and narrow nocheck={nocheck}", flush=True)
+    L = ma.load()
+    if nocheck:
+        ret = L.magma_dgetrf_vbatched_max_nocheck(V.d_rows.data_ptr(), V.d_cols.data_ptr(), 600, V.ptr,
+                                                  V.d_ld.data_ptr(), ipiv.ptr, info.data_ptr(), V.count, queue.handle)
+        queue.sync()
+    else:
+        ret = L.magma_dgetrf_vbatched(V.d_rows.data_ptr(), V.d_cols.data_ptr(), V.ptr, V.d_ld.data_ptr(), ipiv.ptr,
+                                      info.data_ptr(), V.count, queue.handle)
+    assert ret == 0
+    assert info.cpu().numpy()[: V.count].tolist() == [0] * V.count
+    got = V.matrices()
+    for i, (m, n) in enumerate(shapes):
+        LUo, ipo, _ = oracle.dgetrf(mats[i], m=m, n=n)
+        assert np.array_equal(ipiv.numpy(i, min(m, n)), ipo) and same(got[i], LUo), (m, n)
