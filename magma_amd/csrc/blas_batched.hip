@@ -540,10 +540,11 @@ __global__ void __launch_bounds__(256) perm_identity_kernel(int n, double **A_ar
 template <bool T, bool U>
 magma_int_t launch_trsv(int n, double **A, int lda, double **x, int incx, bool unit, int count, hipStream_t st)
 {
-    // from order 17 to 512 the register sweeps, where dtrsv's order is dtrsm's:
-    // 20,000 systems of order 64 448 -> 148 us, of order 32 122 -> 85 us; at
-    // order 8 they take 63 us against 40 us here
-    if (n > 16 && incx == 1 && !(T && !U)) {
+    // from order 17 (a full chip: 21) to 512 the register sweeps, where dtrsv's
+    // order is dtrsm's: 20,000 systems of order 64 448 -> 148 us, of order 32
+    // 122 -> 85 us; at order 17 they take 1.12 to 1.18 times the time of the
+    // kernel here, at order 8 63 us against 40
+    if (n > (count > 4096 ? 20 : 16) && incx == 1 && !(T && !U)) {
         const magma_int_t r = launch_trsm_mfma(true, !U, T, unit, n, 1, 1.0, A, lda, x, n, count, st);
         if (r != MAGMA_ERR_NOT_SUPPORTED) return r;
     }
@@ -561,6 +562,25 @@ magma_int_t launch_trsv(int n, double **A, int lda, double **x, int incx, bool u
     return MAGMA_SUCCESS;
 }
 
+// The order up to which a lane per vector is ahead of the register sweeps, which
+// pad a triangle to 16 rows and the vectors to 16 columns.  Measured over both
+// for orders 6 to 40, 1 to 128 vectors and 64 to 20,000 matrices (sweeps / lanes):
+//   up to 4096 items of 16 vectors, where the chip is not full, the chains
+//     compare: order 6 1.1 to 1.4, Left NoTrans order 12 0.9 to 1.1, Left Trans
+//     (a dot product per row) order 16 0.9 to 1.1, Right order 10 0.8 to 0.9;
+//   above, the lanes' use does: with more than 12 vectors an item Left NoTrans
+//     order 12 1.1, 14 0.8; with 8, Left Trans order 20 1.2, 24 1.0; with 4 or
+//     fewer and over 8192 items Left Trans order 40 1.3, Right order 24 1.1.
+// 20,000 of order 2 with 300 vectors, the farthest apart: 104 against 1068 us.
+int lane_loops_up_to(bool left, bool trans, int nv, int count)
+{
+    static const int up_to[4][3] = {{6, 11, 14}, {8, 13, 17}, {11, 15, 20}, {24, 28, 40}};
+    const long items = (long)count * ceil_div(nv, 16);
+    const int each = nv / ceil_div(nv, 16);
+    const int row = items <= 4096 ? 0 : each > 12 ? 1 : each <= 4 && items > 8192 ? 3 : 2;
+    return up_to[row][!left ? 0 : trans ? 2 : 1];
+}
+
 template <char S, char U, char T>
 magma_int_t launch_trsm(int m, int n, double alpha, double **A, int lda, double **B, int ldb, bool unit, int count,
                         hipStream_t st)
@@ -574,9 +594,11 @@ magma_int_t launch_trsm(int m, int n, double alpha, double **A, int lda, double 
     if constexpr (!(U == 'L' && (S == 'L') == (T == 'T'))) {
         // the register sweeps (trsm_mfma.hip) up to order 512: 20,000 x (64, 16
         // vectors) 1583 -> 188 us
-        const magma_int_t r = launch_trsm_mfma(S == 'L', U == 'L', T == 'T', unit, m, n, alpha, A, lda, B, ldb, count,
-                                               st);
-        if (r != MAGMA_ERR_NOT_SUPPORTED) return r;
+        if (L > lane_loops_up_to(S == 'L', T == 'T', nv, count)) {
+            const magma_int_t r = launch_trsm_mfma(S == 'L', U == 'L', T == 'T', unit, m, n, alpha, A, lda, B, ldb,
+                                                   count, st);
+            if (r != MAGMA_ERR_NOT_SUPPORTED) return r;
+        }
     }
     int G = 1;
     while (G < 64 && G < nv) G *= 2;

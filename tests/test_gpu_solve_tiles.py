@@ -198,3 +198,29 @@ def test_unread_values_do_not_leave_the_sweeps(queue, n):
         assert ma.dgetrs_batched(dA, ip, dB, queue) == 0
         X = dB.numpy()
         assert np.isfinite(X).all() and (X[:, 2] == 0).all() and np.signbit(X[:, 2]).any(axis=1).all()
+
+
+@pytest.mark.parametrize("side,uplo,trans", [c for c in TRSM if c not in (("L", "L", "T"), ("R", "L", "N"))])
+@pytest.mark.parametrize("count,nv,orders", [(4, 5, (6, 7, 11, 12, 14, 15)), (4200, 13, (8, 9, 13, 14, 17, 18)),
+                                             (4200, 7, (11, 12, 15, 16, 20, 21)), (8300, 2, (24, 25, 28, 29, 40, 41))])
+def test_trsm_lane_and_sweep(queue, oracle, side, uplo, trans, count, nv, orders):
+    """Either side of the lines between the lane per vector and the sweeps:
+    bitwise the oracle's dtrsm."""
+    import magma_amd as ma
+    rng = np.random.default_rng(count + nv)
+    for order in orders:
+        m, n = (order, nv) if side == "L" else (nv, order)
+        F, _ = factor_batch(rng, 4, order)
+        B = rng.uniform(-1, 1, (4, n, m))
+        reps = -(-count // 4)
+        dA, dB = device(np.tile(F, (reps, 1, 1))[:count], order), device(np.tile(B, (reps, 1, 1))[:count], m)
+        print(f"trsm lanes/sweep {side}{uplo}{trans} order={order} nv={nv} count={count}", flush=True)
+        ma.load().magmablas_dtrsm_batched(ma.MagmaLeft if side == "L" else ma.MagmaRight,
+                                          ma.MagmaUpper if uplo == "U" else ma.MagmaLower,
+                                          ma.MagmaNoTrans if trans == "N" else ma.MagmaTrans, ma.MagmaNonUnit, m, n, 1.0,
+                                          dA.ptr, dA.ld, dB.ptr, dB.ld, count, queue.handle)
+        X = dB.numpy()
+        for s in range(4):
+            want = oracle.dtrsm(side.encode(), uplo.encode(), trans.encode(), b"N", m, n, 1.0, F[s], B[s])
+            assert same(X[s], want), (order, s)
+            assert np.array_equal(X[s::4], np.broadcast_to(X[s], X[s::4].shape)), (order, s)
