@@ -12,7 +12,7 @@
 //             256 x (500, 7 rhs) 1.90 -> 0.22 ms, getrs 8192 x (256, 1 rhs)
 //             1.92 -> 1.15 ms (3.7 TB/s of the factor).
 //   above     one 256-thread workgroup per matrix, up to 8 right-hand sides in
-//             LDS, one barrier per column.
+//             LDS, one barrier per column.  Also the tiniest systems.
 //
 // For the no-transpose L and U solves the order of an entry's terms is the
 // reference BLAS dtrsm loop order, so results are bit-identical to LAPACK's
@@ -197,7 +197,15 @@ constexpr int kSolveMfmaMax = 512;
 static magma_int_t launch_solve(const MatSet &s, char mode, int max_n, hipStream_t st)
 {
     if (s.count <= 0 || max_n <= 0) return MAGMA_SUCCESS;
-    if (max_n <= kSolveMfmaMax) {
+    // A system of two to eight rows and a few right-hand sides fills neither a
+    // tile nor a chain of 16 rows: the kernel below (sweeps / kernel below, 20,000
+    // systems: n 2, 1 and 8 rhs 1.4 to 1.7 and 1.1 to 1.4; n 4, 1 rhs 1.0 to 1.2,
+    // 4 rhs 0.8 to 1.0; n 8, 2 rhs 0.6 to 0.7.  64 systems: n 2, 16 rhs 1.1 to 1.2;
+    // n 4, 8 rhs 1.0 to 1.2; n 6, 8 rhs 0.9 to 1.1; n 8, 4 rhs 0.9 to 1.05).
+    const bool full = s.count > 4096;
+    const bool tiny = !s.n_arr && !s.nrhs_arr && max_n <= (full ? 4 : 8) &&
+                      (long)max_n * s.nrhs <= (full ? 16 : 32);
+    if (max_n <= kSolveMfmaMax && !tiny) {
         const int nchunks = s.nrhs_arr ? 1 : std::max(1, ceil_div(s.nrhs, 16));
         const size_t lds = (size_t)max_n * (sizeof(double) * kTriPitch + sizeof(int));
         const long items = (long)s.count * nchunks;

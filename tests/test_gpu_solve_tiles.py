@@ -224,3 +224,42 @@ def test_trsm_lane_and_sweep(queue, oracle, side, uplo, trans, count, nv, orders
             want = oracle.dtrsm(side.encode(), uplo.encode(), trans.encode(), b"N", m, n, 1.0, F[s], B[s])
             assert same(X[s], want), (order, s)
             assert np.array_equal(X[s::4], np.broadcast_to(X[s], X[s::4].shape)), (order, s)
+
+
+@pytest.mark.parametrize("count", [5, 4100])
+@pytest.mark.parametrize("n,nrhs", [(1, 16), (1, 33), (2, 8), (2, 9), (2, 16), (2, 17), (4, 4), (4, 8), (4, 9), (5, 1), (8, 4),
+                                    (8, 5), (9, 1)])
+def test_tiny_solves(queue, oracle, count, n, nrhs):
+    """Either side of the lines between the tiniest systems' kernel and the
+    sweeps: getrs bitwise the oracle's, its transpose and potrs by the residual."""
+    import magma_amd as ma
+    import torch
+    rng = np.random.default_rng(100 * n + nrhs)
+    LU, ipiv = factor_batch(rng, 5, n)
+    B = rng.uniform(-1, 1, (5, nrhs, n))
+    many = lambda a: np.tile(a, (-(-count // 5),) + (1,) * (a.ndim - 1))[:count]      # noqa: E731
+    ip = ma.IntBatch(count, n)
+    ip.t.copy_(torch.from_numpy(many(ipiv)))
+    print(f"tiny solves n={n} nrhs={nrhs} count={count}", flush=True)
+    for op in ("N", "T", "potrs"):
+        dA, dB = device(many(LU), n + 1), device(many(B), n + 2)
+        if op == "potrs":
+            assert ma.dpotrs_batched(dA, dB, queue, uplo=ma.MagmaLower) == 0
+        else:
+            assert ma.dgetrs_batched(dA, ip, dB, queue, trans=ma.MagmaNoTrans if op == "N" else ma.MagmaTrans) == 0
+        X = dB.numpy()
+        assert bool(dB.t[:, :, n:].isnan().all())
+        for s in range(5):
+            assert np.array_equal(X[s::5], np.broadcast_to(X[s], X[s::5].shape)), (op, s)
+            L = np.tril(LU[s].T, -1) + np.eye(n)
+            A = L @ np.triu(LU[s].T)                # rows in pivot order
+            for k in reversed(range(n)):
+                p = ipiv[s][k] - 1
+                A[[k, p]] = A[[p, k]]
+            if op == "N":
+                assert same(X[s], oracle.dgetrs(LU[s], ipiv[s], B[s])), s
+            elif op == "T":
+                assert oracle.solve_error(A, X[s], B[s]) < 30, s
+            else:
+                C = np.tril(LU[s].T)
+                assert oracle.solve_error(C @ C.T, X[s], B[s]) < 30, s
