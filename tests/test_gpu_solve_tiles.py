@@ -263,3 +263,27 @@ def test_tiny_solves(queue, oracle, count, n, nrhs):
             else:
                 C = np.tril(LU[s].T)
                 assert oracle.solve_error(C @ C.T, X[s], B[s]) < 30, s
+
+
+@pytest.mark.parametrize("n", [1, 2, 4, 5])
+def test_getri_tiny(queue, oracle, n):
+    """Above 4096 matrices of order up to 4: bitwise the oracle's dgetrs on the
+    identity, info of a singular one."""
+    import magma_amd as ma
+    import torch
+    rng = np.random.default_rng(n)
+    count = 4101
+    LU, ipiv = factor_batch(rng, 3, n)
+    LU[1][n // 2, n // 2] = 0.0
+    dA, dI = device(np.tile(LU, (count // 3, 1, 1)), n + 1), ma.DeviceBatch(np.full((count, n, n), 7.0), ld=n + 2)
+    ip = ma.IntBatch(count, n)
+    ip.t.copy_(torch.from_numpy(np.tile(ipiv, (count // 3, 1))))
+    info = torch.full((count,), -1, dtype=torch.int32, device="cuda")
+    print(f"getri tiny n={n}", flush=True)
+    assert ma.load().magma_dgetri_outofplace_batched(n, dA.ptr, dA.ld, ip.ptr, dI.ptr, dI.ld, info.data_ptr(), count,
+                                                     queue.handle) == 0
+    X = dI.numpy()
+    for s in range(3):
+        assert same(X[s], oracle.dgetrs(LU[s], ipiv[s], np.eye(n))), s
+        assert same(X[s::3], np.broadcast_to(X[s], X[s::3].shape)), s
+    assert info.cpu().numpy().reshape(-1, 3).tolist() == [[0, n // 2 + 1, 0]] * (count // 3)
