@@ -46,9 +46,9 @@ magma_int_t launch_getrf(const MatSet &s, int max_m, int max_n, bool fused_solve
     if (dim <= kRegMax) return launch_getrf_small(s, dim, fused_solve, st);
     // A side of at most 16 leaves the MFMA kernel's block column half empty and,
     // above 128 rows, its LDS holds one or two workgroups per CU: the VALU kernel
-    // (MFMA -> VALU, us: 8 x 512 x 4882 1094 -> 262, 16 x 128 x 8000 515 -> 351,
-    // 300 x 16 x 4166 374 -> 213; but 128 x 16 x 8000 222 -> 262, 512 x 32 x 1220
-    // 221 -> 336, 32 x 512 x 1220 440 -> 623).
+    // (MFMA -> VALU, us: 8 x 512 x 4882 785 -> 262, 16 x 128 x 8000 426 -> 351,
+    // 300 x 16 x 4166 375 -> 213; but 128 x 16 x 8000 224 -> 262, 512 x 32 x 1220
+    // 221 -> 336, 32 x 512 x 1220 271 -> 623).
     const bool narrow = std::min(max_m, max_n) <= 16 && (max_m <= 16 || max_m > 128);
     magma_int_t r = (dim <= kMfmaMax && !narrow) ? launch_getrf_mfma(s, dim, max_m, st)
                                                  : launch_getrf_blocked(s, max_m, st);

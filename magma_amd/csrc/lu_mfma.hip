@@ -20,7 +20,9 @@
 //           slot, a barrier, the workgroup's pivot from the slots (DPP again),
 //           the pivot row and its reciprocal to LDS, a barrier, and the rank-1
 //           update with the pivot row's entries as DPP operands.
-//   store   the block column, finished U rows included, in physical row order.
+//   store   the block column, finished U rows included, in physical row order;
+//           past the last pivot (wide matrices) in the final one (2441 of
+//           32 x 256 401 -> 279 us, 1041 of 64 x 300 426 -> 343 us).
 //
 // What bounds it: the chain of a panel column (about 1500 cycles, half of them
 // the two LDS round trips) and, with the chip full, the bytes.  Why
@@ -428,9 +430,13 @@ __global__ void __launch_bounds__(MT) __attribute__((amdgpu_waves_per_eu(2))) ge
                 pos = pos0;
                 info = info0;
                 reference_block<MT>(sm, A, lda, m, j0, jb, nc, min(j0, mn), pos, info);
-            } else {
+            }
+            // Past the last pivot (m < n) every row's place is known, and the block
+            // column goes there at once.
+            if (!exact || jb == 0) {
+                const int from = jb > 0 ? tid : sm.prow[min(tid, m - 1)];
 #pragma unroll
-                for (int k = 0; k < PW; ++k) a[k] = sm.P[k][tid];
+                for (int k = 0; k < PW; ++k) a[k] = sm.P[k][from];
                 store_rows(j0, a);
             }
             if (jb > 0) {
@@ -441,7 +447,7 @@ __global__ void __launch_bounds__(MT) __attribute__((amdgpu_waves_per_eu(2))) ge
             __syncthreads();
         }
 
-        // LAPACK's row order: every column once through P
+        // LAPACK's row order: every other column once through P
         double a[PW];
         auto load_rows = [&](int c0) {
             GDoublePtr pa = opaque(A + c0 * lda + min(tid, m - 1));
@@ -453,14 +459,14 @@ __global__ void __launch_bounds__(MT) __attribute__((amdgpu_waves_per_eu(2))) ge
         };
         load_rows(0);
 #pragma unroll 1
-        for (int p = 0; p < nblk; ++p) {
+        for (int p = 0; p < npan; ++p) {
             const int c0 = PW * p;
             if (tid < m) {
 #pragma unroll
                 for (int k = 0; k < PW; ++k) sm.P[k][pos] = a[k];
             }
             __syncthreads();
-            if (p + 1 < nblk) load_rows(c0 + PW);
+            if (p + 1 < npan) load_rows(c0 + PW);
             double o[PW];
 #pragma unroll
             for (int k = 0; k < PW; ++k) o[k] = sm.P[k][tid];
@@ -493,7 +499,7 @@ static magma_int_t launch_mt(const MatSet &s, int variant, hipStream_t st)
 // 64 < max_dim <= 512 (the largest m or n); returns MAGMA_ERR_NOT_SUPPORTED
 // above.  The kernel goes by the rows, which are what a workgroup's threads and
 // LDS hold; by the larger side, wide matrices left most of both idle (us:
-// 100 x 512 x 390 1003 -> 595, 64 x 300 x 1041 981 -> 426).
+// 100 x 512 x 390 1003 -> 519, 64 x 300 x 1041 981 -> 343).
 magma_int_t launch_getrf_mfma(const MatSet &s, int max_dim, int max_m, hipStream_t st)
 {
     if (s.count <= 0) return MAGMA_SUCCESS;

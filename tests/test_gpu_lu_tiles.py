@@ -144,3 +144,26 @@ def test_getrf_vbatched_wide_and_narrow(queue, oracle, nocheck):
     for i, (m, n) in enumerate(shapes):
         LUo, ipo, _ = oracle.dgetrf(mats[i], m=m, n=n)
         assert np.array_equal(ipiv.numpy(i, min(m, n)), ipo) and same(got[i], LUo), (m, n)
+
+
+@pytest.mark.parametrize("m,n", [(33, 160), (70, 200), (128, 300), (200, 420)])
+def test_getrf_special_wide(queue, oracle, m, n):
+    """Block columns past the last pivot, which go to the rows' final places at
+    once: after a fallback in the square part, in one of their own, and with
+    an overflow in their updates."""
+    import magma_amd as ma
+    rng = np.random.default_rng(m)
+    A = rng.uniform(-1, 1, (5, n, m))
+    A[1][m // 2, m // 3] = np.nan                    # storage (column, row)
+    A[2][m + 40, 7], A[2][n - 1, m - 1] = np.inf, np.nan
+    A[3] = rng.integers(-2, 3, size=(n, m)) * 1e300
+    A[4][:, 5] = 0.0                                 # a zero row: zeros in U under the fallback's skip
+    A[4][n - 3, 2] = np.inf
+    print(f"getrf wide m={m} n={n}", flush=True)
+    dA = ma.DeviceBatch(A, ld=m + 1)
+    ret, ipiv, info = ma.dgetrf_batched(dA, queue, m=m, n=n)
+    assert ret == 0
+    got, ip, inf = dA.numpy(), ipiv.numpy(), info.cpu().numpy()
+    for s in range(5):
+        LUo, ipo, info_o = oracle.dgetrf(A[s], m=m, n=n)
+        assert inf[s] == info_o and np.array_equal(ip[s], ipo) and same(got[s], LUo), s
