@@ -80,9 +80,9 @@ magma_int_t magma_dsposv_vbatched(magma_uplo_t uplo, magma_int_t *n, magma_int_t
  * variant of every family on the queue's device with synthetic matrices of
  * each size class and keeps the fastest.  Untuned entries use variant 0.
  * Families and their variants:
- *   0 LU, 64 < n <= 512: 0 MFMA kernel, 1 the same at one workgroup per CU,
- *     2 VALU blocked kernel, 3 / 4 register-resident kernel at three / two
- *     workgroups per CU (size class 4, n <= 128, only);
+ *   0 LU, 64 < n <= 512: 0 as many workgroups per CU as fit, 1 one per CU;
+ *     2, and in size class 4 (n <= 128) 3 and 4, are accepted from tables saved
+ *     with earlier versions and mean 0;
  *   1 mixed-precision solver: five variants for n <= 256, two above;
  *   2 DGEMM: 0 32x32, 1 16x16, 2 48x48 tiles per wavefront, 3 64x64 tiles
  *     per workgroup staged through LDS.

@@ -6,7 +6,8 @@
 // routine (dtrsv.f, dtrsm.f, dgemv.f; the testers compare against them,
 // testing/testing_ztrsv_batched.cpp:192, testing/testing_ztrsm_batched.cpp:234,
 // testing/testing_zgemv_batched.cpp:155), each update one fma, so results are
-// bitwise those of the CPU restatement in the oracle.  The reference instead
+// bitwise those of the CPU restatement in the oracle (up to the sign of a zero
+// where the register sweeps of trsm_mfma.hip run).  The reference instead
 // inverts diagonal blocks and multiplies (magmablas/ztrsm_batched.cpp:168-480,
 // magmablas/ztrsv_batched.cu:70-296), which rounds differently; LAPACK's
 // order is the target here.
@@ -19,12 +20,15 @@
 //         Lower), so no case needs a serial dot.  The pivots' columns (rows,
 //         transposed) of A are staged in LDS a panel at a time with coalesced
 //         loads.
+//   Of both, the cases whose terms come in the order of a sweep run on the
+//   register sweeps from the orders on that launch_trsv and lane_loops_up_to
+//   give, up to order 512; the others here:
 //   trsm  one lane per independent vector (a column of B for side Left, a
 //         row for Right), each lane running dtrsm.f's loops for its vector,
 //         held in LDS when it is at most 128 long; matrices with fewer than
 //         64 vectors share a wavefront.  A's entries are the same for every
-//         lane of a matrix, so they are broadcast loads.  Two cases (Left/Trans/Lower and Right/NoTrans/
-//         Lower) add dot products in the order opposite to the order their
+//         lane of a matrix, so they are broadcast loads.  Two cases
+//         (Left/Trans/Lower and Right/NoTrans/Lower) add dot products in the order opposite to the order their
 //         terms become final, which rules out a parallel right-looking form
 //         for bit-exact results.
 //   gemv  NoTrans: one thread per entry of y, columns in order (coalesced A
@@ -892,7 +896,7 @@ magma_int_t magma_dgeqrf_batched(magma_int_t m, magma_int_t n, double **dA_array
     }
     hipStream_t st = stream_of(queue);
     if (batchCount == 0) return MAGMA_SUCCESS;
-    // the matrix fits the registers of one to four wavefronts (9.40 -> 0.86 ms at
+    // the matrix fits the registers of one to four wavefronts (9.40 -> 0.89 ms at
     // order 64, qr_reg.hip)
     if (m > 0 && n > 0 && m <= 128 && n <= 128) {
         magma_int_t r = launch_geqrf_reg(m, n, dA_array, lda, dtau_array, info_array, batchCount, st);

@@ -13,12 +13,15 @@
 //           wavefronts and there is no barrier between columns.
 //   store   the rows of the block column.
 //
-// What bounds it: the panel's chain, about 350 cycles a column (square root,
-// reciprocal, the first update), and below it the bytes.  The form before, a
-// right-looking panel of 16 columns with three barriers per column and the
-// trailing matrix rewritten per panel: 2000 of order 149 0.606 -> 0.383 ms, 4096 of
-// order 128 0.849 -> 0.354 ms, 256 of order 512 3.57 -> 0.95 ms, one of order 256
-// 0.42 -> 0.135 ms.
+// What bounds it: the panel's chain (square root, reciprocal, the first update
+// of a column) and, with three wavefronts per SIMD, their vector issue: at order
+// 149 a wavefront waits 0.44 of its time, waits to issue 0.33 and issues VALU
+// work 0.19 of it, about half of that work the diagonal block that every
+// wavefront factors for itself; the matrix cores are 18% busy.  The form before,
+// a right-looking panel of 16 columns with three barriers per column and the
+// trailing matrix rewritten per panel: 2000 of order 149 0.606 -> 0.369 ms, 4096 of
+// order 128 0.849 -> 0.350 ms, 256 of order 512 3.57 -> 0.955 ms, one of order 256
+// 0.42 -> 0.125 ms.
 //
 // Replaces the reference's lg Cholesky (src/zpotrf_batched.cpp:20-221) for
 // these sizes with one launch.
@@ -128,8 +131,8 @@ __device__ __forceinline__ void right_columns(double (&e)[16], double (&b)[16], 
 
 // At 192 rows the LDS leaves room for three workgroups per CU but 206 registers
 // only for two: there the panel goes in two halves of 16 columns and the update
-// in steps of 8, which takes 152 (2000 of order 149 0.437 -> 0.383 ms, of order
-// 192 0.530 -> 0.472 ms).  At 128, 256 and 512 rows the LDS holds no more
+// in steps of 8, which takes 150 (2000 of order 149 0.437 -> 0.383 ms, of order
+// 192 0.530 -> 0.472 ms; 0.369 at order 149 since each row's updates are one statement).  At 128, 256 and 512 rows the LDS holds no more
 // wavefronts than two per SIMD anyway, and the halves cost 3%.
 template <int MT> constexpr bool three_per_simd() { return MT == 192; }
 

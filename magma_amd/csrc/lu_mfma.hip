@@ -24,8 +24,10 @@
 //           past the last pivot (wide matrices) in the final one (2441 of
 //           32 x 256 401 -> 279 us, 1041 of 64 x 300 426 -> 343 us).
 //
-// What bounds it: the chain of a panel column (about 1500 cycles, half of them
-// the two LDS round trips) and, with the chip full, the bytes.  Why
+// What bounds it: the chain of a panel column (the search, a barrier and an LDS
+// round trip, twice) and, with the chip full, the bytes: 8192 of order 256 move
+// 35.3 GB at 4.0 TB/s, a wavefront waits 0.49 of its time and waits to issue
+// 0.29, and the matrix cores are 19% busy.  Why
 // left-looking with fixed rows: a right-looking form reads and writes the
 // trailing matrix per panel, moves 64 scattered rows of it, and needs passes of
 // its own for the gather, the U solve and the deferred interchanges of L.  The
@@ -35,8 +37,8 @@
 // barriers per column: every wavefront's candidate row written before the
 // first one kept the LDS busy for 450 cycles a column.
 // Measured, getrf alone, right-looking form before: 8192 of order 256 12.85 ms
-// -> 8.88 ms, 256 of order 500 7.5 -> 2.03 ms; 4096 of order 96 0.94 ms (a
-// register-resident kernel for n <= 128) -> 0.67 ms.
+// -> 8.80 ms, 256 of order 500 7.5 -> 1.96 ms; 4096 of order 96 0.94 ms (a
+// register-resident kernel for n <= 128) -> 0.68 ms.
 //
 // Replaces the reference's launch chain for these sizes (panel + laswp + trsm
 // + gemm, src/zgetrf_batched.cpp:222-351, src/zgetrf_panel_batched.cpp:127-243,

@@ -18,8 +18,8 @@
 // dot, update) on two wavefronts per SIMD.  A workgroup per matrix with the
 // matrix in LDS, which this replaces at these sizes, spent its time in the two
 // workgroup reductions and four barriers of each column: 20,000 matrices of
-// order 64 took 9.40 ms, and take 0.86 ms here (1.5 TB/s of the 1.32 GB that
-// has to move).  At 128 the grid of four wavefronts still holds the matrix
+// order 64 took 9.40 ms, and take 0.89 ms here (1.5 TB/s of the 1.32 GB that
+// has to move; a wavefront issues VALU work 0.42 of its time and waits 0.20).  At 128 the grid of four wavefronts still holds the matrix
 // (64 doubles a lane); above, the workgroup kernel of blas_batched.hip runs.
 //
 // Numerics: netlib dgeqr2's reflectors (dlarfg's beta = -sign(alpha)

@@ -8,15 +8,15 @@
 //             or four wavefronts: the sweeps of tri_mfma.h.
 //             The 512 rows are what four wavefronts hold beside the factor
 //             tiles in flight (256 registers a lane).  Against the kernel below
-//             at its sizes: potrs 2000 x (149, 16 rhs) 1.13 -> 0.27 ms, getrs
-//             256 x (500, 7 rhs) 1.90 -> 0.22 ms, getrs 8192 x (256, 1 rhs)
-//             1.92 -> 1.15 ms (3.7 TB/s of the factor).
+//             at its sizes: potrs 2000 x (149, 16 rhs) 1.13 -> 0.18 ms, getrs
+//             256 x (500, 7 rhs) 1.90 -> 0.25 ms, getrs 8192 x (256, 1 rhs)
+//             1.92 -> 1.19 ms (3.6 TB/s of the factor).
 //   above     one 256-thread workgroup per matrix, up to 8 right-hand sides in
 //             LDS, one barrier per column.  Also the tiniest systems.
 //
 // For the no-transpose L and U solves the order of an entry's terms is the
-// reference BLAS dtrsm loop order, so results are bit-identical to LAPACK's
-// dgetrs / dpotrs forward sweep; the transposed sweeps associate their sums in
+// reference BLAS dtrsm loop order, so results are bit-identical (in the register
+// sweeps up to the sign of a zero) to LAPACK's dgetrs / dpotrs forward sweep; the transposed sweeps associate their sums in
 // the opposite order to dtrsm's dot-product form and agree to rounding.
 #include <algorithm>
 #include <type_traits>

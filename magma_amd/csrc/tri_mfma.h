@@ -21,10 +21,13 @@
 //
 // Rounding: an entry gets its terms as single fmas in the order of the solved
 // rows (the MFMA applies its four k terms as the sequential chain), then the
-// division: the reference BLAS order of the forward cases.  The reference's
-// skip of a zero x_k (or zero factor entry) can change a result only where the
-// other operand is not finite, and then the result here is not finite either:
-// callers test that and redo such a matrix with the reference loops.
+// division: the reference BLAS order of the forward cases, and its bits up to
+// the sign of a zero: the reference skips a zero x_k, which keeps its sign, and
+// here it is divided and updated like any other (the inverse of -I has -0 off
+// its diagonal).  Beyond that the skip (or that of a zero factor entry) can
+// change a result only where the other operand is not finite, and then the
+// result here is not finite either: callers test that and redo such a matrix
+// with the reference loops.
 #pragma once
 
 #include "dpp_fma.h"

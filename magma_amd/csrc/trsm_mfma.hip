@@ -4,7 +4,7 @@
 // magmablas_dtrsm_batched: six of its eight side / triangle / transpose cases
 // (Left: not Trans with Lower; Right: not NoTrans with Lower).  In these the
 // terms of an entry become final in the order in which the reference BLAS adds
-// them, so the sweep gives its bits; the other two add the newest term first
+// them, so the sweep gives its bits (up to the sign of a zero); the other two add the newest term first
 // and stay with the lane-per-vector loops of blas_batched.hip.  Right-hand
 // sides are the columns of B (Left) or its rows (Right), 16 to a work item.
 //
@@ -14,8 +14,9 @@
 //
 // Bound: at order 64 the chain of the 4 x 4 triangles (one wavefront per 16
 // vectors), with the factor read once per 16 vectors.  20,000 matrices of order
-// 64: trsm with 16 vectors 1583 -> 188 us (3.5 TB/s of the 0.66 GB that has to
-// move), the inverse 10.7 -> 0.82 ms.
+// 64: trsm with 16 vectors 1583 -> 185 us (3.6 TB/s of the 0.66 GB that has to
+// move), the inverse 10.7 -> 0.81 ms.  Small triangles, and few vectors in large
+// batches, stay with the lane-per-vector loops: blas_batched.hip draws the line.
 #include <algorithm>
 
 #include "kernels.h"
